@@ -19,14 +19,18 @@
 //   * LDS serves ~one 64-lane read instruction per 3 ns per CU.
 //
 // Work decomposition
-//   block  = 8 waves, 128 query rows of one (b, h): 4 row waves x 2 key
-//            halves. Row wave r owns rows [32 r, +32); key half h streams the
-//            64-key tiles 2 k + h its rows can see. The halves keep separate
-//            online-softmax states and merge them through LDS at the end, so a
-//            block's critical path is half its key range.
-//   CU     = one block (160 KiB LDS, <= 256 VGPRs per lane): each SIMD runs
-//            the two waves of one row wave, one per key half.
-//   grid   = persistent blocks of up to two units each. A unit is an item
+//   block  = 128 query rows of one (b, h): 4 row waves x HALVES key halves.
+//            Row wave r owns rows [32 r, +32). Two halves (8 waves, small
+//            grids): key half h streams the 64-key tiles 2 k + h its rows can
+//            see; the halves keep separate online-softmax states and merge
+//            them through LDS at the end, so a block's critical path is half
+//            its key range. One half (4 waves, large grids): one stream of
+//            every tile and no merge. The host picks (use_one_half).
+//   CU     = one two-half block (160 KiB LDS) or two one-half blocks (72 KiB
+//            each), <= 256 VGPRs per lane: each SIMD runs two waves, one per
+//            key half or one of each block.
+//   grid   = one half: a block per item, heaviest first. Two halves:
+//            persistent blocks of up to two units each. A unit is an item
 //            (b, h, 128-row query tile) or one of the two key chunks of a
 //            split item. Without a plan, block b takes item b, then item
 //            G + mirror(b), items numbered heaviest (last) query tile first,
@@ -34,7 +38,7 @@
 //            stay on the block's XCD; with a plan (the host's unit table,
 //            when the items do not fill the chip evenly and a workspace is
 //            given) block b takes the two units the table assigns it.
-//   LDS    = the block's Q tile, plus per key half a 4-stage K ring and a
+//   LDS    = the block's Q tile (two halves), plus per key half a 4-stage K ring and a
 //            5-stage V ring of 64-key tiles, all row-major with 16-byte
 //            chunks XOR-swizzled per row, filled by direct global->LDS loads
 //            (global_load_lds_dwordx4) four tiles ahead of use.
@@ -108,8 +112,16 @@
 // r / l^2 <= 0.03 show fp32-output errors <= 2.17e-4 (error up to ~1.5e-3 x
 // sqrt(r / l^2)); N(0,1) inputs at 1/sqrt(D) stay below 0.013 and take the
 // single-rounding pass only.
+// The two halves of a block each hold their own exact key; one-half blocks
+// have one per row. Root-mean-square error of the fp32 output against float64
+// (relative, N(0,1)): 512 keys 1.69e-4 two halves, 1.78e-4 one half; 1024 keys
+// 1.78e-4, 1.93e-4; 4096 keys 1.98e-4, 2.02e-4; head_dim 128, 1733 keys
+// causal 9.4e-5, 9.9e-5; of the fp16 output 2.68e-4, 2.73e-4; 2.73e-4,
+// 2.83e-4; 2.87e-4, 2.89e-4; 2.22e-4, 2.24e-4. Both rest on the same rounded
+// mass and bound.
 
 #include <algorithm>
+#include <climits>
 #include <map>
 #include <mutex>
 #include <tuple>
@@ -118,6 +130,7 @@
 
 #include "fa_internal.h"
 #include "mfma_tile.h"
+#include "prefill_common.h"
 
 // This file is compiled once per head size: FA_PREFILL_D = 64 gives the
 // head_dim 64 kernels and the shared host entry points, FA_PREFILL_D = 128
@@ -131,32 +144,12 @@ namespace fa {
 namespace {
 
 constexpr int kRowWaves = 4;                  // row waves per key half
-constexpr int kWaves = 2 * kRowWaves;         // x 2 key halves
-constexpr int kThreads = kWaves * kWave;      // 512
 constexpr int kRowsPerWave = 32;
 constexpr int kBr = kRowWaves * kRowsPerWave; // 128 query rows per block
 constexpr int kKStages = 4;
 constexpr int kVStages = 5;
 constexpr int kAhead = 4;                     // tiles in flight ahead of use
 constexpr int kLoadsPerTile = 4;              // global_load_lds per thread per tile
-constexpr int kSplitPRowsBelow = 256;  // rows with fewer keys than this: split P
-// A block is recomputed with split P when, for one of its rows, the squared
-// normalised weights that took a single fp16 rounding sum to more than this
-// (see the precision note at the top of the file).
-constexpr float kRedoRoundedMassAbove = 0.03f;
-// |scale| * sqrt(D) above this (1 is the standard 1/sqrt(D)): rows are peaky
-// from the scale alone, so the first (single-rounding) pass is skipped.
-[[maybe_unused]] constexpr float kSplitAllWidth = 1.5f;  // used by the head_dim 64 build
-constexpr float kNegHuge = -3.0e38f;
-// The max that P is taken against moves only when a row's tile max exceeds it
-// by more than this (log2 units), so P <= 2^8 and O is rescaled on few steps...
-constexpr float kLazyMaxSlack = 8.0f;
-// ...or when the tile max's weight exceeds this fraction of the row sum so
-// far: a key that carries a large share of its row is then taken at the exact
-// max, where its P = 1 is exact and leaves the rounded mass.
-constexpr float kLazyMaxDominant = 1.0f / 16;
-constexpr int kLazyMaxRowsFrom = 1024;  // keys a row sees (at least) to take the lazy max
-
 // Tile geometry for head_dim D (64 or 128). A K or V tile is always 8 KiB:
 // 64 keys of 128 B rows for D = 64, 32 keys of 256 B rows for D = 128, so a
 // step is 16 MFMAs either way (D = 64: QK 2 key blocks x 4 d-steps, PV 4
@@ -172,17 +165,26 @@ struct Geo {
   static constexpr int kChunks = D / 8;            // 16-byte chunks per row
   static constexpr int kRowsPerLoad = kWave / kChunks;  // rows per wave load
   static constexpr int kTileHalves = kBc * D;      // 4096 halves = 8 KiB
-  // D = 64 stages the Q tile in LDS; D = 128 loads Q^T straight into
-  // registers, which leaves the whole LDS to the two rings.
-  static constexpr bool kQInLds = D == 64;
-  // LDS (halves): [Q: 128 rows x 64 (D = 64 only)] [half 0: K ring | V ring] [half 1: ...]
-  static constexpr int kQHalves = kQInLds ? kBr * D : 0;                  // 16 KiB / 0
-  static constexpr int kHalfHalves = (kKStages + kVStages) * kTileHalves; // 72 KiB
-  static constexpr int kLdsHalves = kQHalves + 2 * kHalfHalves;           // 160 / 144 KiB
-  // Half-merge exchange at the end: [row wave][group][64 lanes][4] fp32, the
-  // groups holding the O^T values, then (m, l, r, unused); 16 B per lane and
-  // group, so each group is one conflict-free ds_write_b128 / ds_read_b128.
-  static constexpr int kXchg = 16 * kDB + 4;  // floats per lane
+};
+
+// The block of head_dim D with HALVES key streams (see "Work decomposition").
+template <int D, int HALVES>
+struct Blk : Geo<D> {
+  static_assert(HALVES == 1 || HALVES == 2, "one or two key streams");
+  using G = Geo<D>;
+  static constexpr int kThreads = HALVES * kRowWaves * kWave;  // 256 or 512
+  // D = 64 with two halves stages the Q tile in LDS; the others load Q^T
+  // straight into registers, which leaves the whole LDS to the rings.
+  static constexpr bool kQInLds = D == 64 && HALVES == 2;
+  // LDS (halves): [Q: 128 rows x 64 (if staged)] [half 0: K ring | V ring] [half 1: ...]
+  static constexpr int kQHalves = kQInLds ? kBr * D : 0;                     // 16 KiB / 0
+  static constexpr int kHalfHalves = (kKStages + kVStages) * G::kTileHalves; // 72 KiB
+  static constexpr int kLdsHalves = kQHalves + HALVES * kHalfHalves;  // 160 / 144 / 72 KiB
+  // Exchange area at the end: per row wave [group][64 lanes][4] fp32. Two
+  // halves: the groups hold the O^T values, then (m, l, r, unused); 16 B per
+  // lane and group, so each group is one conflict-free ds_write_b128 /
+  // ds_read_b128. One half: only the wave's verdict.
+  static constexpr int kXchg = HALVES == 2 ? 16 * G::kDB + 4 : 4;  // floats per lane
   static constexpr int kXchgBytes = kRowWaves * kXchg * kWave * 4;
   // Output staging after the exchange: per row wave, its 32 rows of O,
   // row-major with 16-byte chunks XOR-swizzled by row, so that each lane can
@@ -196,20 +198,6 @@ struct Geo {
 
 [[maybe_unused]] __device__ __forceinline__ half8 lds_b128(const _Float16 *p) {
   return *reinterpret_cast<const half8 *>(p);
-}
-
-// The lane index read afresh from the hardware (v_mbcnt, in volatile asm so
-// that the compiler cannot merge it with the kernel's first lane index). The
-// code after the main loop (masked tail, verdict, epilogue) derives its
-// per-lane values from this instead of from values computed before the loop,
-// which the compiler otherwise keeps live across it: at 256 VGPRs they went
-// to scratch (5 per lane at head_dim 64, 11-15 at 128), each item stored and
-// reloaded them, and their write-backs were 2.5-3.4 MB of a C3 launch's HBM
-// writes (C3 46.2 -> 45.8 us, C2 full 27.1 -> 26.4 us without them).
-__device__ __forceinline__ int fresh_lane() {
-  int l;
-  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
-  return l;
 }
 
 // head_dim 64 sums P rows on the matrix cores (rowsum_mfma); head_dim 128,
@@ -500,19 +488,19 @@ __device__ __forceinline__ void slow_step(const KFrags<D> &kf, const VFrags<D> &
   rowsum_mfma<D>(sel, p_lo, st.lacc);
 }
 
-// The K and V rings of one key half: half h owns tiles 2 k + h (k = 0, 1,
+// The K and V rings of one key half: half h of H owns tiles H k + h (k = 0, 1,
 // ...), in K stage k % kKStages and V stage k % kVStages.
-template <int D>
+template <int D, int HALVES>
 struct HalfRing {
   using G = Geo<D>;
   unsigned kring, vring;  // LDS byte addresses of the two rings
   const _Float16 *kp, *vp;
-  int seq, t0, n_tiles, half;  // this half streams tiles t0 + 2 k + half below n_tiles
+  int seq, t0, n_tiles, half;  // this half streams tiles t0 + HALVES k + half below n_tiles
   unsigned voff[2][2];  // [K|V][row block i]: byte offset of this lane's chunk in a tile
   int row_in_tile[2];
   int lds_off[2];       // row block i of this wave, in halves
 
-  __device__ __forceinline__ int tile(int k) const { return t0 + 2 * k + half; }
+  __device__ __forceinline__ int tile(int k) const { return t0 + HALVES * k + half; }
   __device__ __forceinline__ bool exists(int k) const { return tile(k) < n_tiles; }
   __device__ __forceinline__ unsigned kstage(int k) const {
     return kring + (k % kKStages) * (2 * G::kTileHalves);
@@ -579,50 +567,6 @@ struct HalfRing {
   }
 };
 
-// Block -> (b, h) with XCD affinity. The grid stays in level-major order
-// (every head's heaviest query tile first), and blocks go to the 8 XCDs
-// round-robin (block i on XCD i % 8). Head h is "at home" on XCD h % 8:
-// within a level each XCD fills its positions with its home heads first and
-// the leftover heads take the spare positions in a fixed order, so most of a
-// head's blocks share one XCD's L2 (for 14 heads, 89 % of the blocks).
-__host__ __device__ __forceinline__ int home_head(int i, int n_bh) {
-  const int level = i / n_bh;
-  const int k = i - level * n_bh;
-  const int base = (level * n_bh) & 7;
-  const int x = (base + k) & 7;     // XCD of this block
-  const int d_x = (x - base) & 7;   // first position of XCD x in this level
-  const int r = (k - d_x) >> 3;     // rank of position k among XCD x's
-  const int nhome_x = (n_bh - x + 7) >> 3;
-  if (r < nhome_x) return x + 8 * r;
-  // A spare position: its index among all spares (XCDs in order, then rank)
-  // selects the matching overflow head (XCDs in order, then head rank).
-  int s = r - nhome_x;
-  for (int y = 0; y < x; ++y) {
-    const int npos = (n_bh - ((y - base) & 7) + 7) >> 3;
-    const int nhome = (n_bh - y + 7) >> 3;
-    s += npos > nhome ? npos - nhome : 0;
-  }
-  for (int y = 0; y < 8; ++y) {
-    const int npos = (n_bh - ((y - base) & 7) + 7) >> 3;
-    const int nhome = (n_bh - y + 7) >> 3;
-    const int over = nhome > npos ? nhome - npos : 0;
-    if (s < over) return y + 8 * (npos + s);
-    s -= over;
-  }
-  return 0;  // unreachable: spare positions and overflow heads are equal in number
-}
-
-// Grouped queries: the placement heads of XCD x (x, x + 8, x + 16, ...) are
-// given a contiguous run of query heads, in XCD order, so the query heads
-// that read one K/V head (consecutive indices) mostly share an XCD and its
-// L2 holds one copy of that K/V head.
-__host__ __device__ __forceinline__ int grouped_head(int h, int n_bh) {
-  const int x = h & 7;
-  int start = 0;
-  for (int y = 0; y < x; ++y) start += (n_bh - y + 7) >> 3;
-  return start + (h >> 3);
-}
-
 // Work units and their blocks, planned on the host when the items do not
 // fill the chip evenly (at most two per CU): the heaviest items are split
 // into two key chunks, tiles [0, mid) and [mid, n_tiles) with mid =
@@ -645,13 +589,13 @@ constexpr int kPartOFloats = Geo<D>::kDB * 16 * kWave;
 template <int D>
 constexpr int kPartFloats = kPartOFloats<D> + 2 * kWave;
 
-template <int D, bool CAUSAL, bool OUT_F32>
-__global__ __launch_bounds__(kThreads, 1) void prefill_kernel(
+template <int D, int HALVES, bool CAUSAL, bool OUT_F32>
+__global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
     const _Float16 *__restrict__ q, const _Float16 *__restrict__ k,
     const _Float16 *__restrict__ v, void *__restrict__ o, int seq,
     int n_qtiles, int bh_count, int group, float c_scale, bool negate_q, bool split_all,
     const PrefillPlan plan, float *__restrict__ part, unsigned *__restrict__ counters) {
-  using G = Geo<D>;
+  using G = Blk<D, HALVES>;
   constexpr int kBc = G::kBc;
   constexpr int kKB = G::kKB;
   constexpr int kKS = G::kKS;
@@ -664,11 +608,11 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(
   // Wave-uniform (SGPR) so every stage / row-block address below is scalar.
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int rw = wave & (kRowWaves - 1);  // row wave: rows [32 rw, +32)
-  const int half = wave / kRowWaves;      // key half: tiles 2k + half
+  const int half = HALVES == 2 ? wave / kRowWaves : 0;  // key half: tiles HALVES k + half
   const int col = lane & 31;
   _Float16 *const half_lds = lds + G::kQHalves + half * G::kHalfHalves;
   _Float16 *const q_lds = lds;
-  HalfRing<D> ring;
+  HalfRing<D, HALVES> ring;
   ring.kring = lds_addr(half_lds);
   ring.vring = ring.kring + kKStages * (2 * G::kTileHalves);
   ring.seq = seq;
@@ -737,19 +681,24 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(
   ring.t0 = tb;
   ring.n_tiles = te;
   const int wave_key_end = CAUSAL ? min(seq, qw0 + kRowsPerWave) : seq;
-  // Tiles [0, 2 n_main) need no mask for any row of the block, and all its
-  // rows see >= kSplitPRowsBelow keys: each half runs n_main pipelined steps
-  // on them, then at most one masked pipelined step (n_steps <= n_main + 1
-  // whenever n_main > 0: causal, the diagonal adds two tiles; full, the
-  // ragged tail one). Blocks with short rows take the plain split-P step on
-  // every tile.
+  // All rows of the block see >= kSplitPRowsBelow keys: the half runs n_main
+  // pipelined steps on tiles that need no mask, then one masked pipelined
+  // step (causal diagonal, ragged tail). Two halves: tiles [0, 2 n_main) need
+  // no mask for any row of the block. One half: n_main is the wave's own,
+  // the tiles below its own diagonal (every wave of the block passes the same
+  // n_steps barriers whatever its n_main); head_dim 128 leaves the tiles from
+  // main_end + 2 on to the plain split-P step, as two halves do. Blocks with
+  // short rows take the plain split-P step on every tile.
   const bool static_split = CAUSAL ? q0 < kSplitPRowsBelow : seq < kSplitPRowsBelow;
   // Pass 0 rounds P to fp16 once on rows that see enough keys; blocks whose
   // row sums then show a peaky row run again with split P on every tile.
   const bool short_rows = split_all || static_split;
   const int main_end = short_rows ? 0 : (CAUSAL ? q0 / kBc : seq / kBc);
-  const int n_main = max(0, min(main_end, te) - tb) / 2;
-  const int n_steps = (te - tb + 1) / 2;  // steps of the longer half
+  int wave_main = main_end;  // tiles below it need no mask for the wave's rows
+  if (HALVES == 1 && CAUSAL && !short_rows)
+    wave_main = min(min(qw0, seq) / kBc, D == 64 ? INT_MAX : main_end + 2);
+  const int n_main = max(0, min(wave_main, te) - tb) / HALVES;
+  const int n_steps = (te - tb + HALVES - 1) / HALVES;  // steps of the longer half
   // Rows that see many keys take the lazy max; shorter ones keep m at the
   // exact running max, whose P = 1 key takes no rounding.
   const float slack =
@@ -834,6 +783,7 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(
     wait_loads<0>();
     __builtin_amdgcn_s_barrier();
     float *xbase = reinterpret_cast<float *>(lds) + rw * (G::kXchg * kWave);
+    if constexpr (HALVES == 1) return xbase;
     floatx4 *xg = reinterpret_cast<floatx4 *>(xbase) + lane;  // group i at xg[i * kWave]
     if (half == 1) {
 #pragma unroll
@@ -940,7 +890,8 @@ __global__ __launch_bounds__(kThreads, 1) void prefill_kernel(
     // of the block sees >= kSplitPRowsBelow keys.)
     // (head_dim 128: its 32-key tiles put two masked tiles in each half's
     // range; the second one takes the plain step below.)
-    const bool tail = n_steps >= n_main + 1;
+    const bool tail = n_steps >= n_main + 1 && (HALVES == 2 || D == 64 || !CAUSAL ||
+                                                 n_main < main_end + 2 - tb);
     if (kk < n_main) {  // one more (odd) main step; leaves S_{kk+1} in s_b, P_kk in p_a
       ring.advance(kk);
       note_row_sum(st);
@@ -1335,6 +1286,34 @@ int current_cu_count() {
   return hipGetDevice(&dev) == hipSuccess ? device_cu_count(dev) : 0;
 }
 
+// Whether a grid takes one-half blocks (256 threads, two to a CU) instead of
+// two-half blocks (512 threads, one to a CU). Two halves bring an item to its
+// end in half the steps, which is what few long items need; one half has no
+// half merge, its prologue and epilogue run under the CU's other block, a
+// grid is dealt out item by item (two-half blocks take at most two items
+// each, so 600 items load some CUs with two and some with three), and the two
+// waves of a SIMD wait at different barriers. Measured, one half over two
+// (same box, us per call, B H S D):
+//   more than two items per CU, always: 16 12 512 64 full 38.4 -> 24.1,
+//     8 12 1024 64 causal 40.2 -> 28.9, 3 14 2048 64 causal 58.4 -> 39.3,
+//     2 14 4096 64 causal 98.9 -> 88.9, 2 32 (8 K/V heads) 1733 128 causal
+//     96.0 -> 81.4, 4 12 4096 128 causal 285 -> 255; at 1 14 8192 64 full, 2 %
+//     slower;
+//   one to two items per CU: rows of <= 512 keys always (22 12 128 64 12.6 ->
+//     9.8, 7 12 500 64 causal 15.0 -> 12.5); <= 1024 keys full (3 14 777 64
+//     23.8 -> 22.1), or causal from 1.4 items per CU on (4 12 900 64 19.3 ->
+//     17.5; 3 12 1024 64, 1.1 items, 16.0 -> 18.7 and not taken); longer rows
+//     full from 1.8 items per CU up to 2304 keys (2 14 2100 64 49.0 -> 46.9;
+//     1 12 4096 64, 71 -> 82, not taken), and causal never (1 14 4096 64:
+//     47 -> 57);
+//   at most one item per CU: two halves (4 12 640 64 full 12.9 -> 13.4).
+bool use_one_half(long long items, int seq, bool causal, int cu) {
+  if (cu <= 0 || items <= cu) return false;
+  if (items > 2LL * cu || seq <= 512) return true;
+  if (seq <= 1024) return !causal || 5 * items >= 7LL * cu;
+  return !causal && seq <= 2304 && 5 * items >= 9LL * cu;
+}
+
 template <int D, bool CAUSAL, bool OUT_F32>
 void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
                 int seq, int group, float c_scale, bool negate_q, bool split_all,
@@ -1342,6 +1321,14 @@ void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
   const int n_qtiles = (seq + kBr - 1) / kBr;
   const long long items = static_cast<long long>(bh) * n_qtiles;
   const int cu = current_cu_count();
+  static const PrefillPlan no_plan{0, {}};
+  if (use_one_half(items, seq, CAUSAL, cu)) {
+    hipLaunchKernelGGL((prefill_kernel<D, 1, CAUSAL, OUT_F32>), dim3(static_cast<unsigned>(items)),
+                       dim3(Blk<D, 1>::kThreads), 0, stream, static_cast<const _Float16 *>(q),
+                       static_cast<const _Float16 *>(k), static_cast<const _Float16 *>(v), o, seq,
+                       n_qtiles, bh, group, c_scale, negate_q, split_all, no_plan, nullptr, nullptr);
+    return;
+  }
   // With a plan (and its workspace and counters): one block per CU. Otherwise
   // a block takes a whole CU's LDS and up to two items: one block per CU, or
   // half the items when there are more than two per CU; without a CU count,
@@ -1349,7 +1336,6 @@ void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
   const PlanEntry e = prefill_plan({bh, n_qtiles, seq, CAUSAL ? 1 : 0, Geo<D>::kBc, group, cu});
   unsigned *counters = nullptr;
   const PrefillPlan *plan = nullptr;
-  static const PrefillPlan no_plan{0, {}};
   if (e.plan.n_blocks > 0 && workspace != nullptr && workspace_bytes >= plan_workspace_bytes<D>(e))
     counters = merge_counters(stream, static_cast<size_t>(kRowWaves) * e.n_splits);
   if (counters != nullptr) plan = &e.plan;
@@ -1357,8 +1343,8 @@ void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
       plan != nullptr ? plan->n_blocks
       : cu > 0        ? std::min<long long>(items, std::max<long long>(cu, (items + 1) / 2))
                       : items);
-  hipLaunchKernelGGL((prefill_kernel<D, CAUSAL, OUT_F32>), dim3(blocks),
-                     dim3(kThreads), 0, stream,
+  hipLaunchKernelGGL((prefill_kernel<D, 2, CAUSAL, OUT_F32>), dim3(blocks),
+                     dim3(Blk<D, 2>::kThreads), 0, stream,
                      static_cast<const _Float16 *>(q),
                      static_cast<const _Float16 *>(k),
                      static_cast<const _Float16 *>(v), o, seq, n_qtiles, bh, group,
@@ -1396,13 +1382,13 @@ int prefill_occupancy_d(fa_occupancy_entry *out, int cap, int *n) {
   struct K { const char *name; const void *fn; };
   const K ks[] = {
       {D == 64 ? "prefill_kernel<causal=true>" : "prefill_kernel<causal=true, head_dim=128>",
-       reinterpret_cast<const void *>(prefill_kernel<D, true, false>)},
+       reinterpret_cast<const void *>(prefill_kernel<D, 2, true, false>)},
       {D == 64 ? "prefill_kernel<causal=false>" : "prefill_kernel<causal=false, head_dim=128>",
-       reinterpret_cast<const void *>(prefill_kernel<D, false, false>)},
+       reinterpret_cast<const void *>(prefill_kernel<D, 2, false, false>)},
   };
   for (const K &k : ks) {
     if (*n < cap) {
-      const int rc = fill_occupancy_row(&out[*n], k.name, k.fn, kThreads, 0);
+      const int rc = fill_occupancy_row(&out[*n], k.name, k.fn, Blk<D, 2>::kThreads, 0);
       if (rc != FA_OK) return rc;
     }
     ++*n;
@@ -1427,6 +1413,7 @@ size_t prefill_workspace_bytes(int batch, int heads, int seq, bool causal) {
   const int n_qtiles = (seq + kBr - 1) / kBr;
   const int cu = current_cu_count();
   const int c = causal ? 1 : 0;
+  if (use_one_half(static_cast<long long>(bh) * n_qtiles, seq, causal, cu)) return 0;
   // The number of split items depends on the shape only (not on the K/V
   // grouping, which only permutes the heads among the blocks).
   return std::max(
