@@ -706,6 +706,7 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
 
   half8 qf[kDS];
   SoftmaxState<D> st;
+  bool active_rows = true;  // whether this wave computes (one half: its rows run again)
   auto prologue = [&]() {
     // Q: for D = 64 the tile goes to LDS (16 row blocks of 8 rows, 2 per wave;
     // K swizzle); for D = 128 each lane loads its Q^T fragments (query my_q,
@@ -746,6 +747,7 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
       if (negate_q) qf[s] = -qf[s];
     }
 
+    if (HALVES == 1 && !active_rows) return;
     st.m = kNegHuge;
     st.mt = kNegHuge;
     st.r = 0.f;
@@ -764,7 +766,7 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
     // of tile kk + 4 overwrite its K stage.
     for (int kk = kk0; kk < n_steps; ++kk) {
       const int key0 = ring.tile(kk) * kBc;
-      const bool active = key0 < wave_key_end;
+      const bool active = key0 < wave_key_end && (HALVES == 2 || active_rows);
       KFrags<D> kf;
       VFrags<D> vf;
       if (active) {
@@ -947,6 +949,8 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
       const float r_row = st.r + __shfl_xor(st.r, 32);
       const bool peaky = qw0 + (fresh_lane() & 31) < seq &&
                          r_row > kRedoRoundedMassAbove * l_row * l_row;
+      // (One half: waves without such a row keep what they have.)
+      active_rows = HALVES == 2 || __builtin_amdgcn_ballot_w64(peaky) != 0;
       const float verdict = __builtin_amdgcn_ballot_w64(peaky) != 0 ? 1.0f : 0.0f;
       if (lane == 0) xchg[0] = verdict;
     }
@@ -1438,6 +1442,9 @@ int launch_prefill(const void *q, const void *k, const void *v, void *o,
   if (head_dim == 128)
     launch_d<128>(q, k, v, o, out_f32, bh, seq, group, causal, c_scale, negate_q, split_all,
                   workspace, workspace_bytes, stream);
+  else if (prefill_wide_pays(bh, seq, causal, current_cu_count()))
+    launch_prefill_wide(q, k, v, o, out_f32, bh, seq, group, causal, c_scale, negate_q, split_all,
+                        stream);
   else
     launch_d<64>(q, k, v, o, out_f32, bh, seq, group, causal, c_scale, negate_q, split_all,
                  workspace, workspace_bytes, stream);

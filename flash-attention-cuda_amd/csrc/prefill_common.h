@@ -6,6 +6,13 @@
 
 namespace fa {
 
+// head_dim 64 on large grids, 64 query rows per wave (prefill_wide.hip):
+// whether a shape takes it, and its launch (the arguments of launch_d).
+bool prefill_wide_pays(int bh, int seq, bool causal, int cu);
+void launch_prefill_wide(const void *q, const void *k, const void *v, void *o, bool out_f32,
+                         int bh, int seq, int group, bool causal, float c_scale, bool negate_q,
+                         bool split_all, hipStream_t stream);
+
 namespace {
 
 [[maybe_unused]] constexpr int kSplitPRowsBelow = 256;  // rows with fewer keys than this: split P

@@ -1,7 +1,7 @@
-"""Prefill grids of more than two 128-row items per CU, which run as
-one-half blocks (csrc/prefill.hip, use_one_half): every place a ragged end or
-the causal diagonal can fall in a block's tiles, both head sizes, against the
-oracle."""
+"""Prefill grids of more than two 128-row items per CU: one-half blocks
+(csrc/prefill.hip, use_one_half) and, at head_dim 64, 256-row blocks
+(csrc/prefill_wide.hip, prefill_wide_pays): every place a ragged end or the
+causal diagonal can fall in a block's tiles, against the oracle."""
 
 import numpy as np
 import pytest
@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 BOUND = 2.44e-4  # fp32 output; the fp16 output is its rounding
 
 
-def _check_prefill(batch, heads, kv_heads, seq, d, causal, scale, spread=1.0):
+def _check_prefill(batch, heads, kv_heads, seq, d, causal, scale, spread=1.0, check=None):
     gen = torch.Generator().manual_seed(seq * 10 + d + causal)
     q = (torch.randn(batch, heads, seq, d, generator=gen) * spread).half()
     k = (torch.randn(batch, kv_heads, seq, d, generator=gen) * spread).half()
@@ -24,10 +24,14 @@ def _check_prefill(batch, heads, kv_heads, seq, d, causal, scale, spread=1.0):
     out32 = flashattn_cuda._prefill_gqa_fp32(qd, kd, vd, causal, scale)
     out16 = flashattn_cuda.prefill_gqa(qd, kd, vd, causal, scale)
     torch.cuda.synchronize()
-    ref = oracle.prefill_gqa(q.numpy(), k.numpy(), v.numpy(), causal, scale)
-    err = np.abs(out32.cpu().numpy() - ref).max()
-    assert err <= BOUND, err
     assert torch.equal(out16, out32.half())
+    group = heads // kv_heads
+    # Every K/V head's first query head, or the first, last and a few between.
+    some = sorted({h // group * group for h in (check or range(heads))})
+    ref = oracle.prefill_gqa(q[:, some].numpy(), k[:, [h // group for h in some]].numpy(),
+                             v[:, [h // group for h in some]].numpy(), causal, scale)
+    err = np.abs(out32[:, some].cpu().numpy() - ref).max()
+    assert err <= BOUND, err
 
 
 def _heads_for(seq, per_cu):
@@ -53,3 +57,30 @@ def test_one_half_blocks_options(kind, d):
     scale = {"negative scale": -1.0, "wide scale": 2.4}.get(kind, 1.0) * d ** -0.5
     _check_prefill(1, heads, heads // 2 if kind == "grouped" else heads, 600, d, True, scale,
                    1.5 if kind == "wide inputs" else 1.0)
+
+
+def _wide_case(seq, causal):
+    """Heads that give a grid the 256-row blocks take, and heads to check."""
+    cu = torch.cuda.get_device_properties(0).multi_processor_count
+    tiles = -(-seq // 256)
+    heads = 5 * cu // tiles + 1 if causal else 2 * cu // tiles
+    return heads - heads % 2, [0, 1, heads // 3, heads // 2, heads - 3]
+
+
+@pytest.mark.parametrize("causal,seq", [
+    *[(False, s) for s in (512, 513, 544, 575, 577, 608, 639, 700, 768)],
+    *[(True, s) for s in (2048, 2049, 2079, 2111, 2145, 2240)],
+])
+def test_wide_blocks_at_every_tail(seq, causal):
+    heads, check = _wide_case(seq, causal)
+    _check_prefill(1, heads, heads, seq, 64, causal, 0.125, check=check)
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("kind", ["grouped", "negative scale", "wide scale", "wide inputs"])
+def test_wide_blocks_options(kind, causal):
+    seq = 2090 if causal else 720
+    heads, check = _wide_case(seq, causal)
+    scale = {"negative scale": -0.125, "wide scale": 0.3}.get(kind, 0.125)
+    _check_prefill(1, heads, heads // 2 if kind == "grouped" else heads, seq, 64, causal, scale,
+                   1.5 if kind == "wide inputs" else 1.0, check)
