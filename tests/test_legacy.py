@@ -107,3 +107,17 @@ def test_legacy_rejects_bad_inputs():
     with pytest.raises(RuntimeError, match="legacy kernels expect head_dim == 64"):
         w = torch.randn(8, 32, device="cuda")
         fa.legacy_fused(w, w, w)
+
+
+@requires_gpu
+@pytest.mark.parametrize("fn", FNS)
+@pytest.mark.parametrize("n", [15, 16, 17, 255, 256, 273, 8191, 8192, 8209])
+def test_legacy_block_edges(fn, n):
+    """Row and key counts around the 16-row tiles, the sixteen waves' key
+    shares and the switch to 32-row blocks (8192 rows)."""
+    import flashattn_cuda as fa
+
+    q, k, v = _inputs(n, seed=n)
+    out = getattr(fa, fn)(q.cuda(), k.cuda(), v.cuda())
+    ref = oracle.legacy_attention(q.numpy(), k.numpy(), v.numpy())
+    assert np.abs(out.cpu().numpy() - ref).max() <= TOL
