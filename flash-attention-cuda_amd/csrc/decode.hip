@@ -527,114 +527,148 @@ __global__ __launch_bounds__(W * kWave) void decode_split_fused_kernel(
 }
 
 // Pass 2 (decode.cu:143-175): log-sum-exp merge of the partials of one
-// (b, h). Only the ceil(len / chunk) chunks that hold rows are read (the
+// (b, h). Only the ceil(len / chunk) chunks that hold rows count (the
 // reference skips the others through l <= 0); a sequence with no rows
-// produces zeros. One wave per (b, h): lane s takes partials s, s + 64, ...
-// for the max and the row sum, then lane d accumulates head dim d over the
-// chunks, with the per-chunk weights broadcast from the lane that computed
-// them. The loads of the common case (seq_len, the first 64 (m, l) pairs
-// and the first 8 partial rows) are all issued before any of them is used,
-// so the pass costs about one memory round trip.
-// D threads: lane = threadIdx.x % 64 runs the per-chunk statistics (each wave
-// of a 128-thread block computes them for itself), dim = threadIdx.x is the
-// head dim it accumulates.
-template <int D, bool OUT_F32>
-__global__ __launch_bounds__(D) void decode_merge_kernel(
+// produces zeros. One block of W waves per (b, h): wave w takes chunks w,
+// w + W, ..., eight at a time, lane j of it head dims [j D / 64, +D / 64); the
+// W states meet in LDS. Every lane group of 8 holds the eight (m, l), so their
+// max and sums are three DPP steps. The pass is one memory round trip per 8 W
+// chunks: seq_lens, the (m, l) and the partial rows of the first ones are
+// requested before any is used (the host takes W = 1 to 16 by the number of
+// chunks). One wave for all chunks, 16 at a time and the rest one by one, took
+// 4.0 (6 chunks at most), 4.6 (12) and 6.6 us (86) as a kernel. Per call B1 H28/4
+// L16384 13.7 -> 9.7 us, B1 H32/8 L16384 D128 20.4 -> 17.7.
+template <int D, bool OUT_F32, int W>
+__global__ __launch_bounds__(W * kWave) void decode_merge_kernel(
     const float *__restrict__ part_acc, const float *__restrict__ part_ml,
     const int32_t *__restrict__ seq_lens, void *__restrict__ o, int heads,
     int max_seq, int n_splits, int chunk) {
-  constexpr int kBatch = 16;  // chunks whose partial rows are loaded together
+  constexpr int kBatch = 8;
+  constexpr int kDims = D / kWave;  // head dims per lane (1 or 2)
+  typedef float dims __attribute__((ext_vector_type(kDims)));
+  __shared__ dims s_acc[W][kWave];
+  __shared__ float s_ml[W][2];
   const int bh = blockIdx.x;
   const int lane = threadIdx.x & (kWave - 1);
-  const int dim = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
   const size_t base = static_cast<size_t>(bh) * n_splits;
-  // Issued together, before the number of live chunks is known: seq_len, the
-  // (m, l) of chunk `lane` and head dim `dim` of the first kBatch partials
-  // (slots past the live ones are read, all inside the workspace, and then
-  // discarded by a select).
   const int raw_len = seq_lens[bh / heads];
-  float2 ml = make_float2(kNegBig, 0.f);
-  if (lane < n_splits) ml = *reinterpret_cast<const float2 *>(part_ml + (base + lane) * 2);
-  float x[kBatch];
-  const float *col = part_acc + base * D + dim;
+  const dims *const rows = reinterpret_cast<const dims *>(part_acc + base * D) + lane;
+  const float2 *const mls = reinterpret_cast<const float2 *>(part_ml) + base;
+  // Chunk u of the wave's batch from s0 on; slots past the last one read the
+  // last (all inside the workspace; those past the live ones are discarded by
+  // a select: they were not written in this call and may hold any bits).
+  auto load = [&](int s0, float2 &ml, dims (&x)[kBatch]) {
+    ml = mls[min(s0 + W * (lane & (kBatch - 1)), n_splits - 1)];
 #pragma unroll
-  for (int u = 0; u < kBatch; ++u) x[u] = (u < n_splits) ? col[u * D] : 0.f;
-
+    for (int u = 0; u < kBatch; ++u)
+      x[u] = rows[static_cast<size_t>(min(s0 + W * u, n_splits - 1)) * kWave];
+  };
+  float2 ml;
+  dims x[kBatch];
+  load(wave, ml, x);
   const int len = min(raw_len, max_seq);
   const int n_act = len > 0 ? (len + chunk - 1) / chunk : 0;
-  float m_all = lane < n_act ? ml.x : kNegBig;
-  for (int s = lane + kWave; s < n_act; s += kWave) m_all = fmaxf(m_all, part_ml[(base + s) * 2]);
-  m_all = wave_max(m_all);
-  float l_all = lane < n_act ? ml.y * fast_exp2(ml.x - m_all) : 0.f;
-  for (int s = lane + kWave; s < n_act; s += kWave) {
-    const float2 mls = *reinterpret_cast<const float2 *>(part_ml + (base + s) * 2);
-    l_all = fmaf(mls.y, fast_exp2(mls.x - m_all), l_all);
+  float m = kNegBig, l = 0.f;
+  dims acc = 0.f;
+  for (int s0 = wave; s0 < n_act; s0 += W * kBatch) {
+    if (s0 != wave) load(s0, ml, x);
+    const bool live = s0 + W * (lane & (kBatch - 1)) < n_act;
+    const float ms = live ? ml.x : kNegBig;
+    const float m_new = fmaxf(m, max_lanes8(ms));
+    const float f = fast_exp2(m - m_new);
+    const float w = live ? fast_exp2(ms - m_new) : 0.f;
+    l = l * f + sum_lanes8(live ? ml.y * w : 0.f);
+    acc *= f;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const float wu = __builtin_bit_cast(
+          float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), u));
+      if (s0 + W * u < n_act) acc += x[u] * wu;
+    }
+    m = m_new;
   }
-  l_all = wave_sum(l_all);
+  s_acc[wave][lane] = acc;
+  if (lane == 0) {
+    s_ml[wave][0] = m;
+    s_ml[wave][1] = l;
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  float m_all = s_ml[0][0];
+#pragma unroll
+  for (int v = 1; v < W; ++v) m_all = fmaxf(m_all, s_ml[v][0]);
+  float l_all = 0.f;
+  dims out = 0.f;
+#pragma unroll
+  for (int v = 0; v < W; ++v) {
+    const float f = fast_exp2(s_ml[v][0] - m_all);  // waves without chunks: l = 0, acc = 0
+    l_all = fmaf(s_ml[v][1], f, l_all);
+    out += s_acc[v][lane] * f;
+  }
+#pragma unroll
+  for (int d = 0; d < kDims; ++d) {
+    const float r = l_all > 0.f ? out[d] / l_all : 0.f;
+    const size_t idx = static_cast<size_t>(bh) * D + kDims * lane + d;
+    if (OUT_F32)
+      static_cast<float *>(o)[idx] = r;
+    else
+      static_cast<_Float16 *>(o)[idx] = static_cast<_Float16>(r);
+  }
+}
 
-  float acc = 0.f;
-  for (int s0 = 0; s0 < n_act; s0 += kWave) {
-    const int s = s0 + lane;
-    const float w = (s < n_act) ? fast_exp2((s0 == 0 ? ml.x : part_ml[(base + s) * 2]) - m_all) : 0.f;
-    const int cnt = min(kWave, n_act - s0);
-    int t = 0;
-    if (s0 == 0) {
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) {
-        // Slots past n_act were never written for this call (their chunks
-        // hold no rows) and may hold any bits, NaN included: select them
-        // out rather than multiplying them by a zero weight.
-        const float xu = u < n_act ? x[u] : 0.f;
-        acc = fmaf(xu, __shfl(w, u), acc);
-      }
-      t = kBatch;
-    }
-    for (; t + kBatch <= cnt; t += kBatch) {
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) x[u] = col[(s0 + t + u) * D];
-#pragma unroll
-      for (int u = 0; u < kBatch; ++u) acc = fmaf(x[u], __shfl(w, t + u), acc);
-    }
-    for (; t < cnt; ++t) acc = fmaf(col[(s0 + t) * D], __shfl(w, t), acc);
-  }
-  const float out = (l_all > 0.f) ? acc / l_all : 0.f;
-  const size_t idx = static_cast<size_t>(bh) * D + dim;
-  if (OUT_F32) {
-    static_cast<float *>(o)[idx] = out;
-  } else {
-    static_cast<_Float16 *>(o)[idx] = static_cast<_Float16>(out);
-  }
+template <int D>
+void launch_merge(const float *part_acc, const float *part_ml, const int32_t *seq_lens, void *o,
+                  bool out_f32, size_t bh, int heads, int max_seq, int n_splits, int chunk,
+                  hipStream_t stream) {
+  using Kernel = decltype(&decode_merge_kernel<D, false, 1>);
+  static const Kernel kernels[2][5] = {
+      {decode_merge_kernel<D, false, 1>, decode_merge_kernel<D, false, 2>,
+       decode_merge_kernel<D, false, 4>, decode_merge_kernel<D, false, 8>,
+       decode_merge_kernel<D, false, 16>},
+      {decode_merge_kernel<D, true, 1>, decode_merge_kernel<D, true, 2>,
+       decode_merge_kernel<D, true, 4>, decode_merge_kernel<D, true, 8>,
+       decode_merge_kernel<D, true, 16>}};
+  int i = 0;  // 8 chunks per wave and round trip, up to 16 waves
+  while (i < 4 && n_splits > (8 << i)) ++i;
+  const int w = 1 << i;
+  const Kernel kernel = kernels[out_f32 ? 1 : 0][i];
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(bh)), dim3(w * kWave), 0, stream, part_acc,
+                     part_ml, seq_lens, o, heads, max_seq, n_splits, chunk);
 }
 
 // Grouped-query split pass on the matrix cores (H_kv < H): one wave owns the
 // cache rows [chunk_i * chunk, min(len, (chunk_i + 1) * chunk)) of one
-// (b, K/V head) and up to 32 of the query heads that read it, and writes one
-// partial (m, l, acc[64]) per query head in the layout of the VALU split pass
-// above, so the same merge pass combines them. Per 32-row tile:
-//   S^T = K Q^T   4 x v_mfma_f32_32x32x16_f16, the group's queries as the 32
+// (b, K/V head) and up to 16 QB of the query heads that read it (QB = 1 or 2),
+// and writes one partial (m, l, acc[D]) per query head in the layout of the
+// VALU split pass above, so the same merge pass combines them. Per 32-row tile
+// and block of 16 queries, on v_mfma_f32_16x16x32_f16 (lane l: column l % 16,
+// lane group g = l / 16):
+//   S^T = K Q^T   two 16-row blocks, D / 32 steps each; the queries are the 16
 //                 columns (columns past the group compute zeros, unused);
-//   softmax       per lane: one query column, 16 of the 32 rows (the other 16
-//                 in lane l ^ 32), log2 domain, rows past the chunk -> -inf;
-//   O^T += V^T P^T with P split into fp16 hi + lo parts (4 + 4 MFMAs), so
-//                 the weights are P to ~2^-22 at any logit width. (Rounding P
-//                 once to fp16 and computing a chunk again with split P when
-//                 its rounded mass was too large was 3 % faster on N(0,1)
-//                 inputs but 50 % slower once q and k were 1.5x wider: a
-//                 chunk's weights are normalised over its own rows, so most
-//                 chunks failed the check and ran twice. C5 shape with 2 K/V
-//                 heads: 13.6 -> 14.0 us per call at N(0,1), 20.8 -> 14.0 us
-//                 with q and k x1.5.)
+//   softmax       per lane: one query column, rows 4 g + i of both blocks (the
+//                 others in the lanes l ^ 16, l ^ 32), log2 domain, rows past
+//                 the chunk -> -inf;
+//   O^T += V^T P^T with P split into fp16 hi + lo parts (2 x D / 16 MFMAs), so
+//                 the weights are P to ~2^-22 at any logit width. The 32 rows
+//                 are one step: k-slot 8 g + i is row 4 g + i of the first
+//                 block for i < 4 and of the second for i >= 4, which is how
+//                 the S^T accumulators hold P^T.
+// The products of tile t + 1's S^T are issued before tile t's softmax, so the
+// matrix cores and the LDS reads work beside it: what bounds a chunk is the
+// wave's own serial chain per tile, not memory. (32 x 32 x 16 products, half
+// of whose columns even a group of 16 leaves empty, took twice the matrix-core
+// and softmax work: 0.75 us per tile and wave against 0.5 at head_dim 64, 1.2
+// against 0.74 at 128; per call with the merge below B32 H14/2 L4096 ragged 14.1
+// -> 12.7 us, B8 H32/8 L8191 ragged D128 35.7 -> 32.1, B8 H32/1 L4096 12.7 ->
+// 10.0.)
 // K and V tiles stream through a per-wave LDS ring filled by direct
-// global->LDS loads kGroupAhead tiles ahead (row-major, 16-byte chunks
-// XOR-swizzled, as the prefill kernel's tiles), with the non-temporal hint:
-// each cache row is read once per call (B8 H32/8 L4096 17.7 -> 16.1 us per
-// call, the ragged C5 shape with 2 K/V heads within noise). A block is one wave, so
-// nothing is shared and there is no barrier; the ring sets 5 waves per CU.
-// The MFMA work per row is the same for 1 to 32 queries, so a K/V head is
-// read once for its whole group at HBM speed, where the VALU path above pays
-// the dot products and the P V update once per query.
+// global->LDS loads (row-major, 16-byte chunks XOR-swizzled, as the prefill
+// kernel's tiles), with the non-temporal hint: each cache row is read once per
+// call. A block is one wave, so nothing is shared and there is no barrier; the
+// ring sets 5 waves per CU (3 at head_dim 128).
 constexpr int kGroupTile = 32;                           // cache rows per tile
-constexpr int kGroupCols = 32;                           // queries per wave
+constexpr int kGroupCols = 32;                           // queries per wave, at most
 
 // Ring geometry of the grouped pass for head_dim D. A tile is 32 rows of
 // 2 D bytes (4 KiB at D = 64, 8 KiB at D = 128); the ring depth keeps the
@@ -642,8 +676,7 @@ constexpr int kGroupCols = 32;                           // queries per wave
 // CU) for D = 128.
 template <int D>
 struct GroupGeo {
-  static constexpr int kStages = D == 64 ? 4 : 3;        // ring depth per wave (2..4)
-  static constexpr int kAhead = kStages - 1;             // tiles in flight
+  static constexpr int kStages = D == 64 ? 4 : 3;        // ring depth per wave
   static constexpr int kTileHalves = kGroupTile * D;
   static constexpr int kChunks = D / 8;                  // 16-byte chunks per row
   static constexpr int kRowsPerLoad = kWave / kChunks;   // 8 or 4
@@ -651,6 +684,15 @@ struct GroupGeo {
   static constexpr int kLoads = 2 * kRowBlocks;          // K + V loads per lane per tile
   static constexpr int kWavesPerCu = (160 * 1024) / (2 * kStages * kTileHalves * 2);
 };
+
+// V chunk swizzle of the grouped tiles (a 32-lane transpose-read phase reads
+// the chunk pair {2 d, 2 d + 1} of 8 consecutive rows): 8 distinct 32-byte
+// places in the 256 bytes that two 128-byte rows, or one 256-byte row, span.
+template <int D>
+__device__ __forceinline__ int group_v_swz(int row) {
+  if constexpr (D == 64) return ((row >> 1) & 3) << 1;
+  else return (row & 7) << 1;
+}
 
 // Wait until a ring tile is resident while the `later` (<= K) tiles issued
 // after it, L loads each, may still fly (vmcnt counts at most 63).
@@ -667,86 +709,36 @@ __device__ __forceinline__ void wait_ring(int later) {
   }
 }
 
-// Online softmax and O^T += V^T P^T for one tile whose S^T (raw q.k) is in
-// `sacc`: m is the running max in the log2 domain (scores times c), l this
-// lane's share of the row sum. MASK: rows >= lim of this lane's half are past
-// the chunk end. P goes to the matrix cores as fp16 hi + lo parts (two PV
-// products), so the weights that multiply V are P to ~2^-22 whatever the
-// logit width; l sums the same fp16 values the products consume.
-template <int D, bool MASK>
-__device__ __forceinline__ void group_softmax_pv(floatx16 &sacc, const half8 (&vf)[2][D / 32],
-                                                 int lim, float c, float &m, float &l,
-                                                 floatx16 (&o)[D / 32]) {
-  float mx = -INFINITY;
-#pragma unroll
-  for (int a = 0; a < 16; ++a) {
-    if (MASK && 8 * (a >> 2) + (a & 3) >= lim) sacc[a] = -INFINITY;
-    mx = fmaxf(mx, sacc[a]);
-  }
-  mx = max_lane_pair(mx);  // the tile has a row in range: finite
-  const float m_new = fmaxf(m, mx * c);
-  const float alpha = fast_exp2(m - m_new);
-  m = m_new;
-  const half2 ones = {static_cast<_Float16>(1.0f), static_cast<_Float16>(1.0f)};
-  half8 p_hi[2], p_lo[2];
-  float lsum = 0.f;
-#pragma unroll
-  for (int hs = 0; hs < 2; ++hs)
-#pragma unroll
-    for (int e = 0; e < 8; e += 2) {
-      const float s0 = sacc[8 * hs + e], s1 = sacc[8 * hs + e + 1];
-      float p0 = fast_exp2(fmaf(s0, c, -m_new));
-      float p1 = fast_exp2(fmaf(s1, c, -m_new));
-      if (MASK) {  // -inf * c is NaN when c = 0
-        p0 = (s0 == -INFINITY) ? 0.f : p0;
-        p1 = (s1 == -INFINITY) ? 0.f : p1;
-      }
-      const half2 hi2 = {static_cast<_Float16>(p0), static_cast<_Float16>(p1)};
-      p_hi[hs][e] = hi2[0];
-      p_hi[hs][e + 1] = hi2[1];
-      lsum = __builtin_amdgcn_fdot2(hi2, ones, lsum, false);
-      const half2 lo2 = {static_cast<_Float16>(p0 - static_cast<float>(hi2[0])),
-                         static_cast<_Float16>(p1 - static_cast<float>(hi2[1]))};
-      p_lo[hs][e] = lo2[0];
-      p_lo[hs][e + 1] = lo2[1];
-      lsum = __builtin_amdgcn_fdot2(lo2, ones, lsum, false);
-    }
-  l = fmaf(l, alpha, lsum);
-  // Rescaled on every tile (alpha is 1 where the max did not rise): behind a
-  // wave-uniform branch the accumulators were copied to other registers and
-  // back around it on every tile, which cost as much as the multiplies.
-#pragma unroll
-  for (int db = 0; db < D / 32; ++db)
-#pragma unroll
-    for (int a = 0; a < 16; ++a) o[db][a] *= alpha;
-#pragma unroll
-  for (int hs = 0; hs < 2; ++hs)
-#pragma unroll
-    for (int db = 0; db < D / 32; ++db) {
-      o[db] = mfma(vf[hs][db], p_hi[hs], o[db]);
-      o[db] = mfma(vf[hs][db], p_lo[hs], o[db]);
-    }
+// max(x[l], x[l ^ 16], x[l ^ 32], x[l ^ 48]) for every lane (VALU only, no
+// LDS). As in max_lane_pair the swaps are written in asm: the compiler treats
+// a swap of two equal values as a no-op.
+__device__ __forceinline__ float max_lane_groups(float x) {
+  float a = max_lane_pair(x), b = a;
+  asm volatile(
+      "s_nop 1\n\t"
+      "v_permlane16_swap_b32 %0, %1\n\t"
+      "s_nop 0\n\t"
+      "v_max_f32 %0, %0, %1"
+      : "+v"(a), "+v"(b));
+  return a;
 }
 
-template <int D>
+template <int D, int QB>
 __global__ __launch_bounds__(kWave) void decode_group_kernel(
     const _Float16 *__restrict__ q, const _Float16 *__restrict__ k_cache,
     const _Float16 *__restrict__ v_cache, const int32_t *__restrict__ seq_lens,
     float *__restrict__ part_acc, float *__restrict__ part_ml, int heads, int kv_heads,
     int group, int nq, int max_seq, int n_splits, int n_units, int chunk, float qscale) {
   using G = GroupGeo<D>;
-  constexpr int kGroupStages = G::kStages;
-  constexpr int kGroupAhead = G::kAhead;
-  constexpr int kGroupTileHalves = G::kTileHalves;
-  constexpr int kGroupLoads = G::kLoads;
-  constexpr int kDS = D / 16;  // k-steps of S^T = K Q^T
-  constexpr int kDB = D / 32;  // d-blocks of O^T
-  __shared__ __attribute__((aligned(1024))) _Float16 lds[2 * kGroupStages * kGroupTileHalves];
+  constexpr int kKS = D / 32;  // k-steps of S^T = K Q^T
+  constexpr int kDB = D / 16;  // 16-dim blocks of O^T
+  constexpr int kTileBytes = 2 * G::kTileHalves;
+  __shared__ __attribute__((aligned(1024))) _Float16 lds[2 * G::kStages * G::kTileHalves];
   const int unit = static_cast<int>(blockIdx.x);
   if (unit >= n_units) return;
   const int lane = threadIdx.x;
-  const int col = lane & 31;
-  const int g = lane >> 5;
+  const int col = lane & 15;
+  const int g = lane >> 4;
   // Chunk-major unit order, as the VALU split pass (longest-first dispatch).
   // Within a chunk index the query units rotate by that index: block i runs
   // on XCD i % 8, and with a unit count per chunk that is a multiple of 8
@@ -763,8 +755,8 @@ __global__ __launch_bounds__(kWave) void decode_group_kernel(
   const size_t kv_off = (static_cast<size_t>(qu.b) * kv_heads + qu.kv) * max_seq * D;
   const _Float16 *const kp = k_cache + kv_off;
   const _Float16 *const vp = v_cache + kv_off;
-  _Float16 *const kring = lds;
-  _Float16 *const vring = lds + kGroupStages * kGroupTileHalves;
+  const unsigned kring = lds_addr(lds);
+  const unsigned vring = kring + G::kStages * kTileBytes;
 
   // Loads of tile t: lane = (D / 8) * (row in a row block) + 16-byte chunk;
   // 32 / (512 / D) row blocks each of K and V. Rows past the chunk end are
@@ -776,40 +768,57 @@ __global__ __launch_bounds__(kWave) void decode_group_kernel(
   for (int rb = 0; rb < G::kRowBlocks; ++rb) {
     const int r = rb * G::kRowsPerLoad + rr;  // row inside the tile (tiles start at a multiple of 32)
     src_k[rb] = (c16 ^ k_swz_d<D>(r)) << 3;
-    src_v[rb] = (c16 ^ v_swz_d<D>(r)) << 3;
+    src_v[rb] = (c16 ^ group_v_swz<D>(r)) << 3;
   }
   // The Q^T fragments are requested together with seq_lens (two memory
-  // round trips before the rows arrive, not three): column `col` is query
-  // head h0 + col of the unit (zeros past nq), head dims [(D / 2) g + 8 s,
-  // +8) for k-step s. They are waited for before the ring's first loads: a
-  // Q load still pending inside the loop would make the compiler wait for
-  // every load (ring included) there. (Requesting the chunk's first tile
+  // round trips before the rows arrive, not three): column `col` of block qb
+  // is query head h0 + 16 qb + col of the unit (zeros past nq), head dims
+  // [32 s + 8 g, +8) for k-step s. They are waited for before the ring's first
+  // loads: a Q load still pending inside the loop would make the compiler wait
+  // for every load (ring included) there. (Requesting the chunk's first tile
   // before the length as well cost more than it saved on ragged batches,
   // whose units past a sequence's end would read a tile for nothing: C5
   // shape with 2 K/V heads 15.0 -> 15.7 us.)
   const size_t bh0 = static_cast<size_t>(qu.b) * heads + qu.h0;
-  const int qcol = min(col, nq - 1);  // columns past nq load a valid row, then zero it
-  half8 qf[kDS];
+  half8 qf[QB][kKS];
 #pragma unroll
-  for (int st = 0; st < kDS; ++st)
-    qf[st] = *reinterpret_cast<const half8 *>(q + (bh0 + qcol) * D + (D / 2) * g + 8 * st);
+  for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+    for (int s = 0; s < kKS; ++s)  // columns past nq load a valid row, then zero it
+      qf[qb][s] = *reinterpret_cast<const half8 *>(
+          q + (bh0 + min(16 * qb + col, nq - 1)) * D + 32 * s + 8 * g);
   const int len = min(seq_lens[qu.b], max_seq);
   if (begin >= len) {  // no rows: no partial (the merge skips this chunk)
-    hold(qf);
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) hold(qf[qb]);
     return;
   }
   const int end = min(len, begin + chunk);
   const int n_tiles = (end - begin + kGroupTile - 1) / kGroupTile;
+  auto stage = [&](int t) { return (t % G::kStages) * kTileBytes; };
   auto issue = [&](int t) {
     const int row0 = begin + t * kGroupTile;
-    _Float16 *const ks = kring + (t % kGroupStages) * kGroupTileHalves;
-    _Float16 *const vs = vring + (t % kGroupStages) * kGroupTileHalves;
+    const unsigned ks = kring + stage(t), vs = vring + stage(t);
+    if (row0 + kGroupTile <= end) {
+      // Whole tile: a scalar base plus the lane's fixed offset (of which the
+      // swizzles leave one to four different ones per row block).
+      const _Float16 *const kb = kp + static_cast<size_t>(row0) * D;
+      const _Float16 *const vb = vp + static_cast<size_t>(row0) * D;
+#pragma unroll
+      for (int rb = 0; rb < G::kRowBlocks; ++rb) {
+        global_to_lds16_sbase_nt_at(kb + rb * G::kRowsPerLoad * D,
+                                    2u * static_cast<unsigned>(rr * D + src_k[rb]), ks + rb * 1024);
+        global_to_lds16_sbase_nt_at(vb + rb * G::kRowsPerLoad * D,
+                                    2u * static_cast<unsigned>(rr * D + src_v[rb]), vs + rb * 1024);
+      }
+      return;
+    }
 #pragma unroll
     for (int rb = 0; rb < G::kRowBlocks; ++rb) {
       const size_t row =
           static_cast<size_t>(min(row0 + rb * G::kRowsPerLoad + rr, end - 1)) * D;
-      global_to_lds16_nt(kp + row + src_k[rb], ks + rb * G::kRowsPerLoad * D);
-      global_to_lds16_nt(vp + row + src_v[rb], vs + rb * G::kRowsPerLoad * D);
+      global_to_lds16_nt_at(kp + row + src_k[rb], ks + rb * 1024);
+      global_to_lds16_nt_at(vp + row + src_v[rb], vs + rb * 1024);
     }
   };
   // A negative scale is folded into Q (an exact fp16 negation), so the
@@ -817,81 +826,166 @@ __global__ __launch_bounds__(kWave) void decode_group_kernel(
   // scores.
   const float c_scale = fabsf(qscale);
 #pragma unroll
-  for (int st = 0; st < kDS; ++st) {
-    if (col >= nq) qf[st] = half8{};
-    if (qscale < 0.f) qf[st] = -qf[st];
-    asm volatile("" ::"v"(qf[st]));
-  }
+  for (int qb = 0; qb < QB; ++qb)
 #pragma unroll
-  for (int t = 0; t < kGroupAhead; ++t)
+    for (int s = 0; s < kKS; ++s) {
+      if (16 * qb + col >= nq) qf[qb][s] = half8{};
+      if (qscale < 0.f) qf[qb][s] = -qf[qb][s];
+      asm volatile("" ::"v"(qf[qb][s]));
+    }
+#pragma unroll
+  for (int t = 0; t < G::kStages; ++t)
     if (t < n_tiles) issue(t);
 
-  const FragOffsetsD<D> fo = frag_offsets_d<D>(lane);
-  float m = kNegBig, l = 0.f;
-  floatx16 o[kDB];
+  // LDS offsets (halves) of this lane's fragments in a tile; the second
+  // 16-row block is 16 D halves on.
+  int k_off[kKS], v_off[kDB];
+#pragma unroll
+  for (int s = 0; s < kKS; ++s) k_off[s] = col * D + (((4 * s + g) ^ k_swz_d<D>(col)) << 3);
+  const int v_row = 4 * g + (col >> 2);
 #pragma unroll
   for (int db = 0; db < kDB; ++db)
+    v_off[db] = v_row * D + (((2 * db + ((lane & 3) >> 1)) ^ group_v_swz<D>(v_row)) << 3) +
+                4 * (lane & 1);
+  auto read_k = [&](int t, half8 (&kf)[2][kKS]) {
+    const unsigned base = uniform_lds_u(kring + stage(t));
 #pragma unroll
-    for (int a = 0; a < 16; ++a) o[db][a] = 0.f;
-
-  // The last tile is partial when the chunk's row count is not a multiple of
-  // 32: only that tile is masked.
-  const bool partial_tail = ((end - begin) & (kGroupTile - 1)) != 0;
-  for (int t = 0; t < n_tiles; ++t) {
-    // Tile t resident: the loads of the tiles issued after it (up to
-    // kGroupAhead - 1 of them) may still fly.
-    wait_ring<kGroupAhead - 1, kGroupLoads>(min(kGroupAhead - 1, n_tiles - 1 - t));
-    const _Float16 *const ks = kring + (t % kGroupStages) * kGroupTileHalves;
-    const _Float16 *const vs = vring + (t % kGroupStages) * kGroupTileHalves;
-    half8 kf[kDS];
+    for (int s = 0; s < kKS; ++s) {
+      lds_half *const p = opaque_lds_at(base, k_off[s]);
 #pragma unroll
-    for (int st = 0; st < kDS; ++st) kf[st] = *reinterpret_cast<const half8 *>(ks + fo.k[st]);
-    half8 vf[2][kDB];  // [16-row step][d-block]
+      for (int kb = 0; kb < 2; ++kb)
+        kf[kb][s] = *reinterpret_cast<__attribute__((address_space(3))) const half8 *>(p + kb * 16 * D);
+    }
+  };
+  auto read_v = [&](int t, half8 (&vf)[kDB]) {
+    const unsigned base = uniform_lds_u(vring + stage(t));
 #pragma unroll
     for (int db = 0; db < kDB; ++db) {
-      lds_half *pv = opaque_lds(vs + fo.v[db]);
+      lds_half *const p = opaque_lds_at(base, v_off[db]);
 #pragma unroll
-      for (int hs = 0; hs < 2; ++hs)
+      for (int kb = 0; kb < 2; ++kb) {
+        const half4 v4 = __builtin_bit_cast(
+            half4, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                       (__attribute__((address_space(3))) short4v *)(p + kb * 16 * D)));
 #pragma unroll
-        for (int part = 0; part < 2; ++part) {
-          const short4v r = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (__attribute__((address_space(3))) short4v *)(pv + (16 * hs + 8 * part) * D));
-          const half4 v4 = __builtin_bit_cast(half4, r);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) vf[hs][db][4 * part + e] = v4[e];
-        }
+        for (int e = 0; e < 4; ++e) vf[db][4 * kb + e] = v4[e];
+      }
     }
-    // The stage of tile t - 1 is free (its fragments were consumed): refill
-    // it with tile t + kGroupAhead.
-    if (t + kGroupAhead < n_tiles) issue(t + kGroupAhead);
+  };
+  auto qk = [&](const half8 (&kf)[2][kKS], floatx4 (&s)[QB][2]) {
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) s[qb][kb] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < kKS; ++i)
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int kb = 0; kb < 2; ++kb) s[qb][kb] = mfma16(kf[kb][i], qf[qb][i], s[qb][kb]);
+  };
 
-    floatx16 sacc;
+  float m[QB], l[QB];  // l: this lane's rows
+  floatx4 o[QB][kDB];
 #pragma unroll
-    for (int a = 0; a < 16; ++a) sacc[a] = 0.f;
+  for (int qb = 0; qb < QB; ++qb) {
+    m[qb] = kNegBig;
+    l[qb] = 0.f;
 #pragma unroll
-    for (int st = 0; st < kDS; ++st) sacc = mfma(kf[st], qf[st], sacc);
-    if (partial_tail && t == n_tiles - 1) {
-      // Element a: row 8 (a / 4) + 4 g + a % 4 of the tile.
-      const int lim = end - (begin + t * kGroupTile) - 4 * g;
-      group_softmax_pv<D, true>(sacc, vf, lim, c_scale, m, l, o);
-    } else {
-      group_softmax_pv<D, false>(sacc, vf, 0, c_scale, m, l, o);
-    }
+    for (int db = 0; db < kDB; ++db) o[qb][db] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
-
-  // Lanes l and l ^ 32 hold the two row halves of column col: m is shared,
-  // l adds up; each lane writes its half of the D head dims.
-  l += __shfl_xor(l, 32);
-  if (col < nq) {
-    const size_t slot = (bh0 + col) * n_splits + split;
-    float *const dst = part_acc + slot * D;
+  floatx4 s[QB][2];
+  {
+    wait_ring<G::kStages - 1, G::kLoads>(min(G::kStages - 1, n_tiles - 1));
+    half8 kf[2][kKS];
+    read_k(0, kf);
+    qk(kf, s);
+  }
+  for (int t = 0; t < n_tiles; ++t) {
+    // Tile t + 1 resident: the loads of the tiles issued after it may still fly.
+    if (t + 1 < n_tiles)
+      wait_ring<G::kStages - 2, G::kLoads>(min(G::kStages - 2, n_tiles - 2 - t));
+    half8 vf[kDB], kf[2][kKS];
+    read_v(t, vf);
+    read_k(t + 1, kf);  // (past the last tile: any bits of the ring, and S is not used)
+    floatx4 s_next[QB][2];
+    qk(kf, s_next);
+    // The last tile is partial when the chunk's row count is not a multiple
+    // of 32. Element i of block kb: row 16 kb + 4 g + i of the tile.
+    const int lim = end - begin - t * kGroupTile - 4 * g;
+    const bool mask = end - begin - t * kGroupTile < kGroupTile;
+    half8 p_hi[QB], p_lo[QB];
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb) {
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = s[qb][i >> 2][i & 3];
+      if (mask) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (16 * (i >> 2) + (i & 3) >= lim) x[i] = -INFINITY;
+      }
+      float mx = x[0];
+#pragma unroll
+      for (int i = 1; i < 8; ++i) mx = fmaxf(mx, x[i]);
+      mx = max_lane_groups(mx);  // the tile has a row in range: finite
+      const float m_new = fmaxf(m[qb], mx * c_scale);
+      const float alpha = fast_exp2(m[qb] - m_new);
+      m[qb] = m_new;
+      float p[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) p[i] = fast_exp2(fmaf(x[i], c_scale, -m_new));
+      if (mask) {  // -inf * c is NaN when c = 0
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (16 * (i >> 2) + (i & 3) >= lim) p[i] = 0.f;
+      }
+      l[qb] = fmaf(l[qb], alpha, ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7])));
+#pragma unroll
+      for (int i = 0; i < 8; i += 2) {
+        const half2 hi = {static_cast<_Float16>(p[i]), static_cast<_Float16>(p[i + 1])};
+        p_hi[qb][i] = hi[0];
+        p_hi[qb][i + 1] = hi[1];
+        p_lo[qb][i] = static_cast<_Float16>(p[i] - static_cast<float>(hi[0]));
+        p_lo[qb][i + 1] = static_cast<_Float16>(p[i + 1] - static_cast<float>(hi[1]));
+      }
+      // Rescaled on every tile (alpha is 1 where the max did not rise): behind
+      // a wave-uniform branch the accumulators were copied to other registers
+      // and back around it on every tile, which cost as much as the multiplies.
+#pragma unroll
+      for (int db = 0; db < kDB; ++db)
+#pragma unroll
+        for (int a = 0; a < 4; ++a) o[qb][db][a] *= alpha;
+    }
+    // Every LDS read of stage t is done (K in the previous round): refill it.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (t + G::kStages < n_tiles) issue(t + G::kStages);
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-        *reinterpret_cast<float4 *>(dst + db * 32 + 8 * rb + 4 * g) =
-            make_float4(o[db][4 * rb], o[db][4 * rb + 1], o[db][4 * rb + 2], o[db][4 * rb + 3]);
-    if (g == 0) *reinterpret_cast<float2 *>(part_ml + slot * 2) = make_float2(m, l);
+      for (int qb = 0; qb < QB; ++qb) {
+        o[qb][db] = mfma16(vf[db], p_hi[qb], o[qb][db]);
+        o[qb][db] = mfma16(vf[db], p_lo[qb], o[qb][db]);
+      }
+#pragma unroll
+    for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+      for (int kb = 0; kb < 2; ++kb) s[qb][kb] = s_next[qb][kb];
+  }
+
+  // The four lanes of a column hold its row groups: m is shared, l adds up;
+  // each lane writes its quarter of the D head dims.
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb) {
+    l[qb] += __shfl_xor(l[qb], 16);
+    l[qb] += __shfl_xor(l[qb], 32);
+    if (16 * qb + col < nq) {
+      const size_t slot = (bh0 + 16 * qb + col) * n_splits + split;
+      float *const dst = part_acc + slot * D + 4 * g;
+#pragma unroll
+      for (int db = 0; db < kDB; ++db) *reinterpret_cast<floatx4 *>(dst + 16 * db) = o[qb][db];
+      if (g == 0) *reinterpret_cast<float2 *>(part_ml + slot * 2) = make_float2(m[qb], l[qb]);
+    }
   }
 }
 
@@ -1199,17 +1293,23 @@ int decode_group_chunk(int batch, int units_per_row, int max_seq, int head_dim) 
       head_dim == 128 ? GroupGeo<128>::kWavesPerCu : GroupGeo<64>::kWavesPerCu;
   const long long waves = static_cast<long long>(per_cu) * (cu > 0 ? cu : 256);
   const long long work = static_cast<long long>(max_seq) * batch * units_per_row;
-  // head_dim 64: chunks 1.25x the one-round share, and at least 5 tiles: a
-  // wave's first tile arrives ~2 us after it starts and every chunk adds a
-  // partial to merge, so fewer, longer chunks win (measured per call: B32
-  // H14/2 L4096 ragged 15.8 -> 14.5 us, B8 H32/8 L4096 22.2 -> 19.4, B16
-  // H14/2 L2048 13.0 -> 10.1, B1 H32/8 L8192 12.1 -> 11.6, B4 H28/4 L16384
-  // 15.4 -> 15.6). head_dim 128 keeps the one-round share.
-  const bool d64 = head_dim != 128;
-  long long rows = d64 ? (5 * work + 4 * waves - 1) / (4 * waves) : (work + waves - 1) / waves;
+  // Chunks of at least 128 rows, and longer than the one-round share where
+  // that is short: a wave's first tile arrives ~2 us after it starts and every
+  // chunk adds a partial to merge. head_dim 64: 1.25x the share (us per call,
+  // chunk: B32 H14/2 L4096 ragged 160 rows 14.2, 256 12.7, 512 14.7; B1 H14/2
+  // L4096 96 rows 7.0, 128 7.0, 160 7.5, 256 9.1; B32 H32/8 L4096 640 31.5, 1024
+  // 30.8). head_dim 128: 1.5x a share of up to 384 rows (B1 H32/8 L16384 192
+  // rows 17.9, 256 16.2, 384 17.8; B2 H32/8 L16384 all full 352 26.4, 512
+  // 25.4; B1 H28/4 L16384 96 14.9, 128 12.9), else the share (B8 H32/8 L8191
+  // ragged 704 32.1, 1024 32.3, all full 45.9, 44.1).
+  long long rows = (work + waves - 1) / waves;
+  if (head_dim != 128)
+    rows = (5 * work + 4 * waves - 1) / (4 * waves);
+  else if (rows <= 384)
+    rows += rows / 2;
   rows = ((rows + kGroupTile - 1) / kGroupTile) * kGroupTile;
   const long long cap = ((static_cast<long long>(max_seq) + kGroupTile - 1) / kGroupTile) * kGroupTile;
-  rows = std::max<long long>(rows, (d64 ? 5 : 2) * kGroupTile);
+  rows = std::max<long long>(rows, 4 * kGroupTile);
   return static_cast<int>(std::min(rows, std::max<long long>(cap, 2 * kGroupTile)));
 }
 
@@ -1308,15 +1408,8 @@ int launch_valu_decode(const void *q, const void *k_cache, const void *v_cache,
   rc = check_hip(hipGetLastError(), "decode_split_kernel launch");
   if (rc != FA_OK) return rc;
 
-  if (out_f32) {
-    hipLaunchKernelGGL((decode_merge_kernel<D, true>), dim3(static_cast<unsigned>(bh)),
-                       dim3(D), 0, stream, part_acc, part_ml, seq_lens,
-                       o, heads, max_seq, n_splits, split_size);
-  } else {
-    hipLaunchKernelGGL((decode_merge_kernel<D, false>), dim3(static_cast<unsigned>(bh)),
-                       dim3(D), 0, stream, part_acc, part_ml, seq_lens,
-                       o, heads, max_seq, n_splits, split_size);
-  }
+  launch_merge<D>(part_acc, part_ml, seq_lens, o, out_f32, bh, heads, max_seq, n_splits, split_size,
+                  stream);
   return check_hip(hipGetLastError(), "decode_merge_kernel launch");
 }
 
@@ -1333,21 +1426,17 @@ int launch_group_decode(const void *q, const void *k_cache, const void *v_cache,
   const size_t n_gu = n_qg * n_sp;
   float *part_acc = workspace;
   float *part_ml = workspace + static_cast<size_t>(batch) * heads * n_sp * D;
-  hipLaunchKernelGGL((decode_group_kernel<D>), dim3(static_cast<unsigned>(n_gu)), dim3(kWave),
-                     0, stream, static_cast<const _Float16 *>(q),
+  const auto kernel = nqg <= 16 ? decode_group_kernel<D, 1> : decode_group_kernel<D, 2>;
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(n_gu)), dim3(kWave), 0, stream,
+                     static_cast<const _Float16 *>(q),
                      static_cast<const _Float16 *>(k_cache),
                      static_cast<const _Float16 *>(v_cache), seq_lens, part_acc, part_ml,
                      heads, kv_heads, group, nqg, max_seq, n_sp, static_cast<int>(n_gu),
                      split_size, scale * kLog2e);
   int rc = check_hip(hipGetLastError(), "decode_group_kernel launch");
   if (rc != FA_OK) return rc;
-  const unsigned n_bh = static_cast<unsigned>(static_cast<size_t>(batch) * heads);
-  if (out_f32)
-    hipLaunchKernelGGL((decode_merge_kernel<D, true>), dim3(n_bh), dim3(D), 0, stream,
-                       part_acc, part_ml, seq_lens, o, heads, max_seq, n_sp, split_size);
-  else
-    hipLaunchKernelGGL((decode_merge_kernel<D, false>), dim3(n_bh), dim3(D), 0, stream,
-                       part_acc, part_ml, seq_lens, o, heads, max_seq, n_sp, split_size);
+  launch_merge<D>(part_acc, part_ml, seq_lens, o, out_f32, static_cast<size_t>(batch) * heads, heads,
+                  max_seq, n_sp, split_size, stream);
   return check_hip(hipGetLastError(), "decode_merge_kernel launch");
 }
 
@@ -1384,10 +1473,10 @@ int decode_occupancy(fa_occupancy_entry *out, int cap, int *n) {
       {"decode_split_kernel", reinterpret_cast<const void *>(decode_split_kernel<64>),
        kSplitThreads},
       {"decode_merge_kernel",
-       reinterpret_cast<const void *>(decode_merge_kernel<64, false>), kHeadDim},
+       reinterpret_cast<const void *>(decode_merge_kernel<64, false, 4>), 4 * kWave},
       {"decode_bh_kernel", reinterpret_cast<const void *>(decode_bh_kernel<64, false>),
        kBhThreads},
-      {"decode_group_kernel", reinterpret_cast<const void *>(decode_group_kernel<64>), kWave},
+      {"decode_group_kernel", reinterpret_cast<const void *>(decode_group_kernel<64, 1>), kWave},
       {"decode_split_fused_kernel<head_dim=128, waves=4>",
        reinterpret_cast<const void *>(decode_split_fused_kernel<128, false, 4>), 4 * kWave},
       {"decode_split_fused_kernel<head_dim=128, waves=2>",
@@ -1395,11 +1484,11 @@ int decode_occupancy(fa_occupancy_entry *out, int cap, int *n) {
       {"decode_split_kernel<head_dim=128>",
        reinterpret_cast<const void *>(decode_split_kernel<128>), kSplitThreads},
       {"decode_merge_kernel<head_dim=128>",
-       reinterpret_cast<const void *>(decode_merge_kernel<128, false>), 128},
+       reinterpret_cast<const void *>(decode_merge_kernel<128, false, 4>), 4 * kWave},
       {"decode_bh_kernel<head_dim=128>",
        reinterpret_cast<const void *>(decode_bh_kernel<128, false>), kBhThreads},
       {"decode_group_kernel<head_dim=128>",
-       reinterpret_cast<const void *>(decode_group_kernel<128>), kWave},
+       reinterpret_cast<const void *>(decode_group_kernel<128, 1>), kWave},
   };
   for (const K &k : ks) {
     if (*n < cap) {

@@ -310,6 +310,11 @@ int decode_impl(const void *q, const void *k_cache, const void *v_cache,
   const bool auto_split = split_size == 0;
   rc = resolve_split(batch, heads, kv_heads, max_seq, head_dim, &split_size);
   if (rc != FA_OK) return rc;
+  // The fixed scratch takes every grouped shape that fits it at chunks of 160
+  // rows, also where the automatic choice is 128.
+  if (scratch_ws && auto_split && kv_heads != heads && split_size < 160 && max_seq > 160 &&
+      decode_ws_bytes(batch, heads, max_seq, head_dim, split_size) > workspace_bytes)
+    split_size = 160;
   const size_t n_splits = (static_cast<size_t>(max_seq) + split_size - 1) / split_size;
   if (static_cast<size_t>(batch) * heads * n_splits > 0x7fffffffull)
     return set_error(FA_ERR_INVALID_ARGUMENT, "too many split blocks");

@@ -353,3 +353,20 @@ def test_capi_decode_gqa_matches_python_api(capi):
     assert rc == 0, capi.fa_last_error()
     torch.cuda.synchronize()
     assert torch.equal(o, flashattn_cuda.decode_gqa(q, k, v, lens, SCALE))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("heads,kv_heads", [(2, 1), (15, 1), (16, 1), (17, 1), (32, 2), (26, 1)])
+@pytest.mark.parametrize("max_seq,split", [(31, 0), (33, 32), (700, 32), (1050, 64), (2100, 32), (4200, 32)])
+def test_decode_gqa_column_blocks_and_merge_widths(heads, kv_heads, d, max_seq, split):
+    """One and two 16-query column blocks per wave, and a merge of 1 to 132
+    chunks (one to sixteen waves, one and more rounds), against the oracle
+    (weights split to 2^-22: an fp32-grade bound)."""
+    gen = torch.Generator().manual_seed(heads * max_seq + d)
+    lens = torch.tensor([max_seq, max(1, max_seq - 33), 1], dtype=torch.int32)
+    q = torch.randn(3, heads, 1, d, generator=gen).half()
+    k = torch.randn(3, kv_heads, max_seq, d, generator=gen).half()
+    v = torch.randn(3, kv_heads, max_seq, d, generator=gen).half()
+    out = flashattn_cuda._decode_gqa_fp32(q.cuda(), k.cuda(), v.cuda(), lens.cuda(), d ** -0.5, split)
+    ref = oracle.decode_gqa(q.numpy(), k.numpy(), v.numpy(), lens.numpy(), d ** -0.5)
+    assert np.abs(out.cpu().numpy() - ref).max() <= 5e-6

@@ -154,3 +154,13 @@ def test_noalloc_first_call_inside_graph_capture():
                          text=True, timeout=300)
     print(res.stdout, res.stderr[-2000:])
     assert res.returncode == 0 and "ok" in res.stdout
+
+
+def test_noalloc_grouped_takes_longer_chunks_where_the_automatic_ones_do_not_fit(lib):
+    """The automatic chunk (128 rows here) needs 8.65 MB of partials, 160-row
+    chunks 6.9 MB: the call runs with those, as an explicit split of 160 does."""
+    q, k, v, lens = _inputs(4, 32, 1, 32768, 64, seed=5)
+    assert lib.fa_decode_hd_workspace_bytes(4, 32, 1, 32768, 64, 0) > SCRATCH_BYTES
+    got = _run(lib, True, q, k, v, lens, FA_OUT_F32, 1, 0.125, 0)
+    want = _run(lib, False, q, k, v, lens, FA_OUT_F32, 1, 0.125, 160)
+    assert torch.equal(got, want)
