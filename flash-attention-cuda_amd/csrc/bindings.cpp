@@ -24,6 +24,7 @@
 
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/hip/HIPCachingAllocator.h>
 
 #include <cmath>
 #include <string>
@@ -57,6 +58,20 @@ void *stream_of(const at::Tensor &t) {
   return static_cast<void *>(
       c10::hip::getCurrentHIPStreamMasqueradingAsCUDA(t.device().index()).stream());
 }
+
+// Transient workspace from torch's caching allocator, on the current stream of
+// the current (guarded) device and stream-ordered like a tensor's memory, but
+// without a tensor around it (submitting a B1 H12 L4096 decode 6.1 -> 5.6 us).
+struct Workspace {
+  explicit Workspace(size_t bytes)
+      : ptr(bytes > 0 ? c10::hip::HIPCachingAllocator::raw_alloc(bytes) : nullptr) {}
+  ~Workspace() {
+    if (ptr != nullptr) c10::hip::HIPCachingAllocator::raw_delete(ptr);
+  }
+  Workspace(const Workspace &) = delete;
+  Workspace &operator=(const Workspace &) = delete;
+  void *const ptr;
+};
 
 // bindings.cpp:10-27. With `grouped`, k and v are [B, H_kv, S, 64] with
 // H_kv dividing H (grouped-query attention, no reference counterpart);
@@ -97,9 +112,7 @@ at::Tensor prefill_impl(const at::Tensor &q, const at::Tensor &k,
   const size_t ws_bytes = fa_prefill_workspace_bytes(
       static_cast<int>(q.size(0)), static_cast<int>(q.size(1)),
       static_cast<int>(q.size(2)), causal ? 1 : 0);
-  at::Tensor ws;
-  if (ws_bytes > 0)
-    ws = at::empty({static_cast<int64_t>(ws_bytes)}, q.options().dtype(at::kByte));
+  const Workspace ws(ws_bytes);
   check_status(fa_prefill_hd(q.const_data_ptr(), k.const_data_ptr(),
                              v.const_data_ptr(), o.data_ptr(),
                              out_f32 ? FA_OUT_F32 : FA_OUT_F16,
@@ -108,8 +121,7 @@ at::Tensor prefill_impl(const at::Tensor &q, const at::Tensor &k,
                              static_cast<int>(k.size(1)),
                              static_cast<int>(q.size(2)), static_cast<int>(q.size(3)),
                              causal ? 1 : 0, static_cast<float>(scale),
-                             ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes,
-                             stream_of(q)));
+                             ws.ptr, ws_bytes, stream_of(q)));
   return o;
 }
 
@@ -197,16 +209,13 @@ at::Tensor decode_core(const at::Tensor &q, const at::Tensor &k_cache,
   check_status(ws_bytes > 0 || fa_last_error()[0] == '\0' ? FA_OK : FA_ERR_INVALID_ARGUMENT);
   // Transient, stream-ordered workspace from the caching allocator
   // (decode.cu:215-219 of the reference), only when the split-K partials need it.
-  at::Tensor ws;
-  if (ws_bytes > 0)
-    ws = at::empty({static_cast<int64_t>(ws_bytes / sizeof(float))},
-                   q.options().dtype(at::kFloat));
+  const Workspace ws(ws_bytes);
   check_status(fa_decode_hd(q.const_data_ptr(), k_cache.const_data_ptr(),
                             v_cache.const_data_ptr(),
                             seq_lens.const_data_ptr<int32_t>(), o.data_ptr(),
                             out_f32 ? FA_OUT_F32 : FA_OUT_F16, batch, heads, kv_heads,
                             max_seq, head_dim, static_cast<float>(scale), split,
-                            ws_bytes > 0 ? ws.data_ptr() : nullptr, ws_bytes, stream_of(q)));
+                            ws.ptr, ws_bytes, stream_of(q)));
   return o;
 }
 
