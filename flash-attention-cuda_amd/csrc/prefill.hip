@@ -1318,9 +1318,13 @@ int current_cu_count() {
 //     full from 1.8 items per CU up to 2304 keys (2 14 2100 64 49.0 -> 46.9;
 //     1 12 4096 64, 71 -> 82, not taken), and causal never (1 14 4096 64:
 //     47 -> 57);
-//   at most one item per CU: two halves (4 12 640 64 full 12.9 -> 13.4).
+//   at most one item per CU: two halves (4 12 640 64 full 12.9 -> 13.4), but
+//     sequences of one query tile, whose half merge costs what two streams of
+//     one tile save (1 12 128 64 6.9 -> 6.6, 1 12 128 128 10.2 -> 9.1).
 bool use_one_half(long long items, int seq, bool causal, int cu) {
-  if (cu <= 0 || items <= cu) return false;
+  if (cu <= 0) return false;
+  if (seq <= kBr) return true;
+  if (items <= cu) return false;
   if (items > 2LL * cu || seq <= 512) return true;
   if (seq <= 1024) return !causal || 5 * items >= 7LL * cu;
   return !causal && seq <= 2304 && 5 * items >= 9LL * cu;
