@@ -629,8 +629,10 @@ void launch_merge(const float *part_acc, const float *part_ml, const int32_t *se
       {decode_merge_kernel<D, true, 1>, decode_merge_kernel<D, true, 2>,
        decode_merge_kernel<D, true, 4>, decode_merge_kernel<D, true, 8>,
        decode_merge_kernel<D, true, 16>}};
-  int i = 0;  // 8 chunks per wave and round trip, up to 16 waves
-  while (i < 4 && n_splits > (8 << i)) ++i;
+  // 8 chunks per wave and round trip, up to 16 waves
+  // (fewer where the grid would pass 2^32 - 1 threads).
+  int i = 0;
+  while (i < 4 && n_splits > (8 << i) && bh < (size_t{1} << 25 >> i)) ++i;
   const int w = 1 << i;
   const Kernel kernel = kernels[out_f32 ? 1 : 0][i];
   hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(bh)), dim3(w * kWave), 0, stream, part_acc,

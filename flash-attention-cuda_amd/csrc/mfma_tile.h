@@ -57,23 +57,13 @@ __device__ __forceinline__ void global_to_lds16(const void *src, const void *lds
       : "v"(src), "s"(m0)
       : "memory", "m0");
 }
-// The same load with a wave-uniform 64-bit base in SGPRs and a per-lane
-// 32-bit byte offset (the saddr form): no per-lane address arithmetic.
-__device__ __forceinline__ void global_to_lds16_sbase(const void *base, unsigned voff,
-                                                      const void *lds_dst) {
-  const unsigned m0 = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void *)(lds_dst))));
-  asm volatile(
-      "s_mov_b32 m0, %2\n\t"
-      "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %0, %1"
-      :
-      : "v"(voff), "s"(base), "s"(m0)
-      : "memory", "m0");
-}
-// The same two loads with the LDS destination given as a byte address (a
+// The same load with the LDS destination given as a byte address (a
 // wave-uniform value kept from lds_addr): no generic-to-LDS pointer cast, and
-// so no null check, per load.
+// so no null check, per load. _sbase: a wave-uniform 64-bit base in SGPRs and a
+// per-lane 32-bit byte offset (the saddr form), no per-lane address arithmetic.
+// _nt: the non-temporal hint, for data read exactly once per call (the decode's
+// cache rows): it bypasses the normal cache-allocation policy, as the VALU
+// decode's nontemporal register loads do.
 __device__ __forceinline__ void global_to_lds16_at(const void *src, unsigned lds_dst) {
   const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_dst);
   asm volatile(
@@ -84,9 +74,6 @@ __device__ __forceinline__ void global_to_lds16_at(const void *src, unsigned lds
       : "v"(src), "s"(m0)
       : "memory", "m0");
 }
-// (with the non-temporal hint, for data read exactly once per call (the
-// decode's cache rows): it bypasses the normal cache-allocation policy, as the
-// VALU decode's nontemporal register loads do)
 __device__ __forceinline__ void global_to_lds16_nt_at(const void *src, unsigned lds_dst) {
   const unsigned m0 = __builtin_amdgcn_readfirstlane(lds_dst);
   asm volatile(
@@ -167,35 +154,9 @@ __device__ __forceinline__ half8 rowsum_selector(int lane) {
   return s;
 }
 
-// Per-lane LDS offsets (in halves, relative to a tile) of every fragment a
-// wave reads from a tile; loop invariant.
-struct FragOffsets {
-  int k[4];  // K (and Q) fragment for d-step s (32-key block 0; block 1 is +32 rows)
-  int v[2];  // V^T transpose-read base for d-block db (key sub-blocks add rows)
-};
-
-__device__ __forceinline__ FragOffsets frag_offsets(int lane) {
-  FragOffsets f;
-  const int col = lane & 31;
-  const int g = lane >> 5;
-#pragma unroll
-  for (int s = 0; s < 4; ++s)
-    f.k[s] = col * kHeadDim + (((4 * g + s) ^ k_swz(col)) << 3);
-  // Lane l of a 16-lane group points at row 4 g + (l % 16) / 4 (plus the
-  // 8-key sub-block), head dims [16 ((l / 16) % 2) + 4 (l % 4), +4).
-  const int tr_row = 4 * g + ((lane & 15) >> 2);
-  const int tr_dim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-#pragma unroll
-  for (int db = 0; db < 2; ++db) {
-    const int d = db * 32 + tr_dim;
-    f.v[db] = tr_row * kHeadDim + (((d >> 3) ^ v_swz(tr_row)) << 3) + (d & 7);
-  }
-  return f;
-}
-
-// The same building blocks for tiles of D-dim rows, D in {64, 128}. D = 64 is
-// exactly the layout above. D = 128 rows are 256 B (16 chunks), so a row
-// no longer shifts the bank group of a chunk and the swizzles change:
+// Tiles of D-dim rows, D in {64, 128}. D = 64 takes the swizzles above. D = 128
+// rows are 256 B (16 chunks), so a row no longer shifts the bank group of a
+// chunk and the swizzles change:
 //  K, Q: a ds_read_b128 phase reads one logical chunk of 8 or 16
 //     consecutive rows; chunk c of row r goes to position c ^ (r & 15),
 //     16 distinct positions for any 16 consecutive rows.
@@ -215,6 +176,8 @@ __device__ __forceinline__ int v_swz_d(int row) {
   else return (row & 3) << 2;
 }
 
+// Per-lane LDS offsets (in halves, relative to a tile) of every fragment a
+// wave reads from a tile; loop invariant.
 template <int D>
 struct FragOffsetsD {
   int k[D / 16];  // K (and Q) fragment for d-step s (key block 0; block 1 is +32 rows)
@@ -230,6 +193,8 @@ __device__ __forceinline__ FragOffsetsD<D> frag_offsets_d(int lane) {
 #pragma unroll
   for (int s = 0; s < D / 16; ++s)
     f.k[s] = col * D + ((((D / 16) * g + s) ^ k_swz_d<D>(col)) << 3);
+  // Lane l of a 16-lane group points at row 4 g + (l % 16) / 4 (plus the
+  // 8-key sub-block), head dims [16 ((l / 16) % 2) + 4 (l % 4), +4).
   const int tr_row = 4 * g + ((lane & 15) >> 2);
   const int tr_dim = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
 #pragma unroll
@@ -242,31 +207,17 @@ __device__ __forceinline__ FragOffsetsD<D> frag_offsets_d(int lane) {
 
 typedef __attribute__((address_space(3))) const _Float16 lds_half;
 
-// An LDS address the compiler must materialise as one register per step:
-// the constant row offsets of the reads below then fold into the
-// instructions' offset fields instead of being hoisted out of the loop as
-// separate loop-invariant addresses.
-__device__ __forceinline__ lds_half *opaque_lds(const _Float16 *p) {
-  unsigned a = static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_half *)(p)));
-  asm volatile("" : "+v"(a));
-  return reinterpret_cast<lds_half *>(static_cast<uintptr_t>(a));
-}
-
-// LDS address base + 2 * off_halves, with base a wave-uniform tile address
-// kept whole in an SGPR (so no constant part of it is split off into a
-// separate vector add) and the sum opaque as in opaque_lds.
-__device__ __forceinline__ unsigned uniform_lds_base(const _Float16 *p) {
-  unsigned a = __builtin_amdgcn_readfirstlane(
-      static_cast<unsigned>(reinterpret_cast<uintptr_t>((lds_half *)(p))));
-  asm volatile("" : "+s"(a));
-  return a;
-}
-// uniform_lds_base for a tile already given as an LDS byte address.
+// A wave-uniform LDS byte address kept whole in an SGPR (so no constant part of
+// it is split off into a separate vector add).
 __device__ __forceinline__ unsigned uniform_lds_u(unsigned a) {
   a = __builtin_amdgcn_readfirstlane(a);
   asm volatile("" : "+s"(a));
   return a;
 }
+// LDS address base + 2 * off_halves, which the compiler must materialise as one
+// register per step: the constant row offsets of the reads from it then fold
+// into the instructions' offset fields instead of being hoisted out of the loop
+// as separate loop-invariant addresses.
 __device__ __forceinline__ lds_half *opaque_lds_at(unsigned base, int off_halves) {
   unsigned a = base + 2u * static_cast<unsigned>(off_halves);
   asm volatile("" : "+v"(a));

@@ -591,17 +591,17 @@ constexpr int kPartOFloats = Geo<D>::kDB * 16 * kWave;
 template <int D>
 constexpr int kPartFloats = kPartOFloats<D> + 2 * kWave;
 
-// PLAN is PrefillPlan or NoPlan: launches without a plan leave its 3 KiB out of
+// PLANNED: whether the launch has a plan; others leave its 3 KiB out of
 // the kernel arguments, which the host copies on every call (submitting a B1 H12
 // S128 prefill 6.1 -> 4.9 us, with the plan looked up without copying it).
 struct NoPlan {};
-template <int D, int HALVES, bool CAUSAL, bool OUT_F32, typename PLAN>
+template <int D, bool CAUSAL, bool OUT_F32, int HALVES, bool PLANNED>
 __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
     const _Float16 *__restrict__ q, const _Float16 *__restrict__ k,
     const _Float16 *__restrict__ v, void *__restrict__ o, int seq,
     int n_qtiles, int bh_count, int group, float c_scale, bool negate_q, bool split_all,
-    const PLAN plan, float *__restrict__ part, unsigned *__restrict__ counters) {
-  constexpr bool kPlanned = std::is_same<PLAN, PrefillPlan>::value;
+    const typename std::conditional<PLANNED, PrefillPlan, NoPlan>::type plan,
+    float *__restrict__ part, unsigned *__restrict__ counters) {
   using G = Blk<D, HALVES>;
   constexpr int kBc = G::kBc;
   constexpr int kKB = G::kKB;
@@ -652,7 +652,7 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
 #pragma unroll
   for (int round = 0; round < 2; ++round) {
   int pos, code = 0, split = 0;
-  if constexpr (kPlanned) {
+  if constexpr (PLANNED) {
     const unsigned u = plan.unit[2 * b_id + round];
     if (u == kNoUnit) break;
     pos = static_cast<int>(u & 0xfffffu);
@@ -681,8 +681,8 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
   const int n_tiles = (key_end + kBc - 1) / kBc;
   // This unit's tiles [tb, te): the whole range, or one chunk of it (tb is
   // even, so each half keeps the parity of its tiles).
-  const int tb = kPlanned && code == 2 ? split_mid(n_tiles) : 0;
-  const int te = kPlanned && code == 1 ? split_mid(n_tiles) : n_tiles;
+  const int tb = PLANNED && code == 2 ? split_mid(n_tiles) : 0;
+  const int te = PLANNED && code == 1 ? split_mid(n_tiles) : n_tiles;
   ring.kp = k + kv_off;
   ring.vp = v + kv_off;
   ring.t0 = tb;
@@ -975,7 +975,7 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
   }
   if (half == 1) continue;
 
-  if (kPlanned && code != 0) {
+  if (PLANNED && code != 0) {
     // ---- one chunk of a split item ---------------------------------------------
     // Each row wave publishes its (O, m, l) partial, waits until it is stored
     // and counts itself on the (item, row wave) counter; the second to arrive
@@ -1338,7 +1338,7 @@ void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
   const long long items = static_cast<long long>(bh) * n_qtiles;
   const int cu = current_cu_count();
   if (use_one_half(items, seq, CAUSAL, cu)) {
-    hipLaunchKernelGGL((prefill_kernel<D, 1, CAUSAL, OUT_F32, NoPlan>), dim3(static_cast<unsigned>(items)),
+    hipLaunchKernelGGL((prefill_kernel<D, CAUSAL, OUT_F32, 1, false>), dim3(static_cast<unsigned>(items)),
                        dim3(Blk<D, 1>::kThreads), 0, stream, static_cast<const _Float16 *>(q),
                        static_cast<const _Float16 *>(k), static_cast<const _Float16 *>(v), o, seq,
                        n_qtiles, bh, group, c_scale, negate_q, split_all, NoPlan{}, nullptr, nullptr);
@@ -1356,7 +1356,7 @@ void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
   const auto *kp = static_cast<const _Float16 *>(k);
   const auto *vp = static_cast<const _Float16 *>(v);
   if (counters != nullptr) {
-    hipLaunchKernelGGL((prefill_kernel<D, 2, CAUSAL, OUT_F32, PrefillPlan>),
+    hipLaunchKernelGGL((prefill_kernel<D, CAUSAL, OUT_F32, 2, true>),
                        dim3(static_cast<unsigned>(e->plan.n_blocks)), dim3(Blk<D, 2>::kThreads), 0,
                        stream, qp, kp, vp, o, seq, n_qtiles, bh, group, c_scale, negate_q,
                        split_all, e->plan, static_cast<float *>(workspace), counters);
@@ -1364,7 +1364,7 @@ void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
   }
   const unsigned blocks = static_cast<unsigned>(
       cu > 0 ? std::min<long long>(items, std::max<long long>(cu, (items + 1) / 2)) : items);
-  hipLaunchKernelGGL((prefill_kernel<D, 2, CAUSAL, OUT_F32, NoPlan>), dim3(blocks),
+  hipLaunchKernelGGL((prefill_kernel<D, CAUSAL, OUT_F32, 2, false>), dim3(blocks),
                      dim3(Blk<D, 2>::kThreads), 0, stream, qp, kp, vp, o, seq, n_qtiles, bh, group,
                      c_scale, negate_q, split_all, NoPlan{}, nullptr, nullptr);
 }
@@ -1399,9 +1399,9 @@ int prefill_occupancy_d(fa_occupancy_entry *out, int cap, int *n) {
   struct K { const char *name; const void *fn; };
   const K ks[] = {
       {D == 64 ? "prefill_kernel<causal=true>" : "prefill_kernel<causal=true, head_dim=128>",
-       reinterpret_cast<const void *>(prefill_kernel<D, 2, true, false, NoPlan>)},
+       reinterpret_cast<const void *>(prefill_kernel<D, true, false, 2, false>)},
       {D == 64 ? "prefill_kernel<causal=false>" : "prefill_kernel<causal=false, head_dim=128>",
-       reinterpret_cast<const void *>(prefill_kernel<D, 2, false, false, NoPlan>)},
+       reinterpret_cast<const void *>(prefill_kernel<D, false, false, 2, false>)},
   };
   for (const K &k : ks) {
     if (*n < cap) {
