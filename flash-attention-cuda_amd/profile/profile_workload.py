@@ -40,6 +40,8 @@ WORKLOADS = {
                           "flop", 4.0 * 4 * 12 * 1024 * 1024 * 64 / 2),
     "prefill_c2_full": ("config 2: full prefill B=4 H=12 S=1024", "prefill_kernel<64, false",
                         "flop", 4.0 * 4 * 12 * 1024 * 1024 * 64),
+    "prefill_large": ("full prefill B=8 H=12 S=4096 (64-row waves)", "prefill_wide_kernel<false",
+                      "flop", 4.0 * 8 * 12 * 4096 * 4096 * 64),
     "prefill_c3_d128": ("config 3 shape at head_dim 128: causal prefill B=1 H=14 S=4096 D=128, scale 1/sqrt(128)",
                         "prefill_kernel<128, true", "flop", 4.0 * 14 * 4096 * 4096 * 128 / 2),
     "decode_c4": ("config 4: decode B=1 H=12 L=4096 (split-K, merged in the same launch)",
@@ -138,6 +140,7 @@ RUNNERS = {
     "prefill_c3": lambda: _prefill(1, 14, 4096, True),
     "prefill_c2_causal": lambda: _prefill(4, 12, 1024, True),
     "prefill_c2_full": lambda: _prefill(4, 12, 1024, False),
+    "prefill_large": lambda: _prefill(8, 12, 4096, False),
     "prefill_c3_d128": lambda: _prefill(1, 14, 4096, True, d=128),
     "decode_c4": lambda: _decode(1, 12, 4096, lens=[4096]),
     "decode_c5": lambda: _decode(32, 14, 4096),
