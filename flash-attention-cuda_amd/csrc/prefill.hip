@@ -24,8 +24,10 @@
 //            grids): key half h streams the 64-key tiles 2 k + h its rows can
 //            see; the halves keep separate online-softmax states and merge
 //            them through LDS at the end, so a block's critical path is half
-//            its key range. One half (4 waves, large grids): one stream of
-//            every tile and no merge. The host picks (use_one_half).
+//            its key range. One half (4 waves, large grids): the same two
+//            streams, each with its own state, one after the other through
+//            one ring; O runs on from the first into the second (main_steps).
+//            The host picks (use_one_half).
 //   CU     = one two-half block (160 KiB LDS) or two one-half blocks (72 KiB
 //            each), <= 256 VGPRs per lane: each SIMD runs two waves, one per
 //            key half or one of each block.
@@ -112,13 +114,14 @@
 // r / l^2 <= 0.03 show fp32-output errors <= 2.17e-4 (error up to ~1.5e-3 x
 // sqrt(r / l^2)); N(0,1) inputs at 1/sqrt(D) stay below 0.013 and take the
 // single-rounding pass only.
-// The two halves of a block each hold their own exact key; one-half blocks
-// have one per row. Root-mean-square error of the fp32 output against float64
-// (relative, N(0,1)): 512 keys 1.69e-4 two halves, 1.78e-4 one half; 1024 keys
-// 1.78e-4, 1.93e-4; 4096 keys 1.98e-4, 2.02e-4; head_dim 128, 1733 keys
-// causal 9.4e-5, 9.9e-5; of the fp16 output 2.68e-4, 2.73e-4; 2.73e-4,
-// 2.83e-4; 2.87e-4, 2.89e-4; 2.22e-4, 2.24e-4. Both rest on the same rounded
-// mass and bound.
+// A row's two key halves each hold their own exact key, in both kinds of block.
+// (One running max per row in one-half blocks, one exact key, raised the
+// root-mean-square error of the fp32 output against float64, relative, N(0,1),
+// from 1.84e-4 to 2.00e-4 at 1024 keys, 2.00e-4 to 2.04e-4 at 4096 keys, and at
+// head_dim 128 from 9.4e-5 to 9.9e-5 at 1733 keys causal; of the fp16 output
+// 2.76e-4 to 2.87e-4, 2.88e-4 to 2.90e-4, 2.22e-4 to 2.24e-4. Running only the
+// waves with a peaky row again, not their block, left the other rows' single
+// rounding: 3.8e-7 to 2.8e-5 at 512 keys with q and k x1.5.)
 
 #include <algorithm>
 #include <climits>
@@ -150,6 +153,7 @@ constexpr int kBr = kRowWaves * kRowsPerWave; // 128 query rows per block
 constexpr int kKStages = 4;
 constexpr int kVStages = 5;
 constexpr int kAhead = 4;                     // tiles in flight ahead of use
+constexpr float kCarryMax = 64.0f;            // log2 units (one-half blocks, see main_steps)
 constexpr int kLoadsPerTile = 4;              // global_load_lds per thread per tile
 // Tile geometry for head_dim D (64 or 128). A K or V tile is always 8 KiB:
 // 64 keys of 128 B rows for D = 64, 32 keys of 256 B rows for D = 128, so a
@@ -489,20 +493,29 @@ __device__ __forceinline__ void slow_step(const KFrags<D> &kf, const VFrags<D> &
   rowsum_mfma<D>(sel, p_lo, st.lacc);
 }
 
-// The K and V rings of one key half: half h of H owns tiles H k + h (k = 0, 1,
-// ...), in K stage k % kKStages and V stage k % kVStages.
+// The K and V rings of one key stream, whose step k is in K stage k % kKStages
+// and V stage k % kVStages. Two-half blocks: half h streams tiles 2 k + h.
+// One-half blocks: the even tiles in the first n_first steps, then the odd
+// ones, or (in_order) every tile as it comes.
 template <int D, int HALVES>
 struct HalfRing {
   using G = Geo<D>;
   unsigned kring, vring;  // LDS byte addresses of the two rings
   const _Float16 *kp, *vp;
-  int seq, t0, n_tiles, half;  // this half streams tiles t0 + HALVES k + half below n_tiles
+  int seq, t0, n_tiles, half;  // two halves: tiles t0 + 2 k + half below n_tiles
+  int n_first;                  // one half
+  bool in_order;                // one half
   unsigned voff[2][2];  // [K|V][row block i]: byte offset of this lane's chunk in a tile
   int row_in_tile[2];
   int lds_off[2];       // row block i of this wave, in halves
 
-  __device__ __forceinline__ int tile(int k) const { return t0 + HALVES * k + half; }
-  __device__ __forceinline__ bool exists(int k) const { return tile(k) < n_tiles; }
+  __device__ __forceinline__ int tile(int k) const {
+    if constexpr (HALVES == 2) return t0 + 2 * k + half;
+    return in_order ? k : k < n_first ? 2 * k : 2 * (k - n_first) + 1;
+  }
+  __device__ __forceinline__ bool exists(int k) const {
+    return (HALVES == 2 ? tile(k) : k) < n_tiles;
+  }
   __device__ __forceinline__ unsigned kstage(int k) const {
     return kring + (k % kKStages) * (2 * G::kTileHalves);
   }
@@ -615,7 +628,7 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
   // Wave-uniform (SGPR) so every stage / row-block address below is scalar.
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
   const int rw = wave & (kRowWaves - 1);  // row wave: rows [32 rw, +32)
-  const int half = HALVES == 2 ? wave / kRowWaves : 0;  // key half: tiles HALVES k + half
+  const int half = HALVES == 2 ? wave / kRowWaves : 0;  // key half (two halves)
   const int col = lane & 31;
   _Float16 *const half_lds = lds + G::kQHalves + half * G::kHalfHalves;
   _Float16 *const q_lds = lds;
@@ -649,8 +662,9 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
   const int grid = static_cast<int>(gridDim.x);
   const int b_id = static_cast<int>(blockIdx.x);
   const int b_mirror = (grid & 7) == 0 ? grid - 8 * (b_id / 8 + 1) + (b_id & 7) : grid - 1 - b_id;
+  // (One half: an item per block.)
 #pragma unroll
-  for (int round = 0; round < 2; ++round) {
+  for (int round = 0; round < HALVES; ++round) {
   int pos, code = 0, split = 0;
   if constexpr (PLANNED) {
     const unsigned u = plan.unit[2 * b_id + round];
@@ -688,24 +702,21 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
   ring.t0 = tb;
   ring.n_tiles = te;
   const int wave_key_end = CAUSAL ? min(seq, qw0 + kRowsPerWave) : seq;
-  // All rows of the block see >= kSplitPRowsBelow keys: the half runs n_main
-  // pipelined steps on tiles that need no mask, then one masked pipelined
-  // step (causal diagonal, ragged tail). Two halves: tiles [0, 2 n_main) need
-  // no mask for any row of the block. One half: n_main is the wave's own,
-  // the tiles below its own diagonal (every wave of the block passes the same
-  // n_steps barriers whatever its n_main); head_dim 128 leaves the tiles from
-  // main_end + 2 on to the plain split-P step, as two halves do. Blocks with
-  // short rows take the plain split-P step on every tile.
+  // Tiles [0, 2 n_main) need no mask for any row of the block, and all its
+  // rows see >= kSplitPRowsBelow keys: each half runs n_main pipelined steps
+  // on them, then at most one masked pipelined step (n_steps <= n_main + 1
+  // whenever n_main > 0: causal, the diagonal adds two tiles; full, the
+  // ragged tail one). Blocks with short rows take the plain split-P step on
+  // every tile.
   const bool static_split = CAUSAL ? q0 < kSplitPRowsBelow : seq < kSplitPRowsBelow;
   // Pass 0 rounds P to fp16 once on rows that see enough keys; blocks whose
   // row sums then show a peaky row run again with split P on every tile.
   const bool short_rows = split_all || static_split;
   const int main_end = short_rows ? 0 : (CAUSAL ? q0 / kBc : seq / kBc);
-  int wave_main = main_end;  // tiles below it need no mask for the wave's rows
-  if (HALVES == 1 && CAUSAL && !short_rows)
-    wave_main = min(min(qw0, seq) / kBc, D == 64 ? INT_MAX : main_end + 2);
-  const int n_main = max(0, min(wave_main, te) - tb) / HALVES;
-  const int n_steps = (te - tb + HALVES - 1) / HALVES;  // steps of the longer half
+  const int n_main = max(0, min(main_end, te) - tb) / 2;
+  const int n_steps = (te - tb + 1) / 2;  // steps of the longer half
+  ring.n_first = n_steps;
+  ring.in_order = HALVES == 1 && short_rows;
   // Rows that see many keys take the lazy max; shorter ones keep m at the
   // exact running max, whose P = 1 key takes no rounding.
   const float slack =
@@ -713,7 +724,15 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
 
   half8 qf[kDS];
   SoftmaxState<D> st;
-  bool active_rows = true;  // whether this wave computes (one half: its rows run again)
+  float m_even = kNegHuge;  // one half: the max of the even tiles' weights
+  auto reset_softmax = [&]() {
+    st.m = kNegHuge;
+    st.mt = kNegHuge;
+    st.r = 0.f;
+    st.lprev = 0.f;
+    st.l = 0.f;
+    st.lacc = floatx4{0.f, 0.f, 0.f, 0.f};
+  };
   auto prologue = [&]() {
     // Q: for D = 64 the tile goes to LDS (16 row blocks of 8 rows, 2 per wave;
     // K swizzle); for D = 128 each lane loads its Q^T fragments (query my_q,
@@ -754,26 +773,20 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
       if (negate_q) qf[s] = -qf[s];
     }
 
-    if (HALVES == 1 && !active_rows) return;
-    st.m = kNegHuge;
-    st.mt = kNegHuge;
-    st.r = 0.f;
-    st.lprev = 0.f;
-    st.l = 0.f;
-    st.lacc = floatx4{0.f, 0.f, 0.f, 0.f};
+    reset_softmax();
 #pragma unroll
     for (int db = 0; db < kDB; ++db)
 #pragma unroll
       for (int a = 0; a < 16; ++a) st.o[db][a] = 0.f;
   };
-  auto split_steps = [&](int kk0) {
+  auto split_steps = [&](int kk0, int kk_end) {
     // ---- short-row blocks: one plain split-P step per tile ---------------------
     // Tile kk is resident (waited for by an earlier advance, or by the
     // prologue); its fragments are read before the barrier that lets the load
     // of tile kk + 4 overwrite its K stage.
-    for (int kk = kk0; kk < n_steps; ++kk) {
+    for (int kk = kk0; kk < kk_end; ++kk) {
       const int key0 = ring.tile(kk) * kBc;
-      const bool active = key0 < wave_key_end && (HALVES == 2 || active_rows);
+      const bool active = key0 < wave_key_end;
       KFrags<D> kf;
       VFrags<D> vf;
       if (active) {
@@ -827,7 +840,6 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
     return xbase;
   };
 
-  prologue();
   // ---- pipelined main loop ---------------------------------------------------
   // Step k: MFMAs QK(k+1) [K_{k+1}, read at step k-1] and PV(k-1) [P_{k-1},
   // V_{k-1}] interleave with the softmax of S_k; the first part of QK(k+1)
@@ -835,8 +847,18 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
   // alternate between even and odd steps. QK(k+1) is issued unconditionally:
   // on the last main step it reads whatever K stage k+1 holds (in bounds)
   // and the result is discarded.
-  int kk = 0;
-  if (n_main > 0) {
+  // These are ring steps [k0, k_end): n_main unmasked ones, then the masked
+  // one; returns the first step left to split_steps.
+  // One half, the odd tiles (odd): they take a max and a row sum of their own,
+  // so P is rounded against the same max as in two-half blocks, but O runs on:
+  // it follows from the even tiles' max to the first odd tile's. (A second O,
+  // merged at the end, has no registers: kept in scratch memory it took B2
+  // H32/8 S1733 D128 causal from 90 to 101 us.) Where the odd tiles' max is more
+  // than kCarryMax lower, O could overflow and the odd tiles weigh less than
+  // 2^-kCarryMax: their max starts there instead.
+  auto main_steps = [&](auto odd, int k0, int k_end) {
+    const int k_main = k0 + n_main;
+    int kk = k0;
     floatx16 s_a[kKB], s_b[kKB];
     half8 p_a[kKS], p_b[kKS], p_unused[kKS];
     KFrags<D> kf;
@@ -845,23 +867,31 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
     // its PV. pm_a, pm_b: largest weights of the P tiles in p_a, p_b.
     float alpha, pm_a, pm_b;
     bool rescale;
-    read_k(ring.kstage(0), fo, kf);
+    read_k(ring.kstage(k0), fo, kf);
     qk_mfma(kf, qf, s_a);
-    read_k(ring.kstage(1), fo, kf);
+    read_k(ring.kstage(k0 + 1), fo, kf);
 
-    // step 0 (no PV yet)
-    ring.advance(0);
+    // the first step (no PV yet)
+    ring.advance(k0);
     rescale = tile_max<CAUSAL, false>(s_a, 0, c_scale, slack, st, alpha, pm_a);
+    if constexpr (decltype(odd)::value) {
+      const float m = fmaxf(st.m, m_even - kCarryMax);
+      pm_a = m == st.m ? pm_a : 0.f;
+      st.m = m;
+      st.mt = fmaxf(st.mt, m);
+      alpha = fast_exp2(m_even - m);
+      rescale = true;
+    }
     qk_mfma(kf, qf, s_b);
     tile_exp<false, false>(s_a, c_scale, pm_a, st, p_a, p_unused);
     __builtin_amdgcn_sched_barrier(0);
-    read_k(ring.kstage(2), fo, kf);
-    read_v(ring.vstage(0), fo, vf);
-    kk = 1;
+    read_k(ring.kstage(k0 + 2), fo, kf);
+    read_v(ring.vstage(k0), fo, vf);
+    ++kk;
 
-    // steps kk (odd: S_kk in s_b, P_{kk-1} in p_a) and kk + 1 (even); kf and
+    // steps kk (the half's odd ones: S_kk in s_b, P_{kk-1} in p_a) and kk + 1 (even); kf and
     // vf hold K_{kk+1} and V_{kk-1}.
-    for (; kk + 1 < n_main; kk += 2) {
+    for (; kk + 1 < k_main; kk += 2) {
       ring.wait(kk);
       qk_mfma_part(kf, qf, s_a, 0);
       ring.pass(kk);
@@ -899,9 +929,8 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
     // of the block sees >= kSplitPRowsBelow keys.)
     // (head_dim 128: its 32-key tiles put two masked tiles in each half's
     // range; the second one takes the plain step below.)
-    const bool tail = n_steps >= n_main + 1 && (HALVES == 2 || D == 64 || !CAUSAL ||
-                                                 n_main < main_end + 2 - tb);
-    if (kk < n_main) {  // one more (odd) main step; leaves S_{kk+1} in s_b, P_kk in p_a
+    const bool tail = k_end > k_main;
+    if (kk < k_main) {  // one more (odd) main step; leaves S_{kk+1} in s_b, P_kk in p_a
       ring.advance(kk);
       note_row_sum(st);
       rescale_o(st, alpha, rescale);
@@ -939,39 +968,67 @@ __global__ __launch_bounds__(HALVES * kRowWaves * kWave, 2) void prefill_kernel(
       rowsum_mfma<D>(sel, p_a, st.lacc);
       pv_mfma(vf, p_a, st.o);
     }
-  }
+    return kk;
+  };
 
-  split_steps(kk);
-  float *xchg = merge_halves();
-  if (!short_rows) {
-    // Every row of a half-0 wave now holds its final (l, r). One fp16
-    // rounding of each weight perturbs the output row by about 2^-11 times
-    // the root of the squared normalised weights that took it, r / l^2: a row
-    // that a few keys carry (beyond its exact P = 1 key) has a large r / l^2.
-    // Blocks with such a row run again with split P. Each half-0 wave leaves
-    // its verdict in its own (already consumed) exchange slot; after the
-    // barrier every wave reads all four.
-    if (half == 0) {
-      const float l_row = kMfmaRowSum<D> ? st.lacc[0] : st.l + __shfl_xor(st.l, 32);
-      const float r_row = st.r + __shfl_xor(st.r, 32);
-      const bool peaky = qw0 + (fresh_lane() & 31) < seq &&
-                         r_row > kRedoRoundedMassAbove * l_row * l_row;
-      // (One half: waves without such a row keep what they have.)
-      active_rows = HALVES == 2 || __builtin_amdgcn_ballot_w64(peaky) != 0;
-      const float verdict = __builtin_amdgcn_ballot_w64(peaky) != 0 ? 1.0f : 0.0f;
-      if (lane == 0) xchg[0] = verdict;
-    }
-    __syncthreads();
-    bool redo = false;
+  bool split_pass = HALVES == 1 && short_rows;  // whether a pass with split P is to run
+  if (!split_pass) {
+    prologue();
+    int kk = 0;
+    if constexpr (HALVES == 2) {
+      if (n_main > 0) kk = main_steps(std::false_type{}, 0, n_steps);
+      split_steps(kk, n_steps);
+    } else {
+      // Both halves in turn, through one ring: the last steps of the even
+      // tiles issue the loads of the first odd ones.
+      kk = main_steps(std::false_type{}, 0, n_steps);
+      if constexpr (D == 128) split_steps(kk, n_steps);
+      m_even = st.m;
+      const float l_even = kMfmaRowSum<D> ? st.lacc[0] : st.l, r_even = st.r;
+      reset_softmax();
+      kk = main_steps(std::true_type{}, n_steps, n_tiles);
+      if constexpr (D == 128) split_steps(kk, n_tiles);
+      const float m = fmaxf(m_even, st.m);
+      const float f0 = fast_exp2(m_even - m), f1 = fast_exp2(st.m - m);
 #pragma unroll
-    for (int r = 0; r < kRowWaves; ++r)
-      redo = redo || reinterpret_cast<const float *>(lds)[r * (G::kXchg * kWave)] != 0.0f;
-    if (redo) {
-      __syncthreads();  // every wave has read the verdicts before the LDS is reloaded
-      prologue();
-      split_steps(0);
-      merge_halves();
+      for (int db = 0; db < kDB; ++db)
+#pragma unroll
+        for (int a = 0; a < 16; ++a) st.o[db][a] *= f1;
+      if constexpr (kMfmaRowSum<D>)
+        st.lacc[0] = l_even * f0 + st.lacc[0] * f1;
+      else
+        st.l = l_even * f0 + st.l * f1;
+      st.r = r_even * (f0 * f0) + st.r * (f1 * f1);
     }
+    float *xchg = merge_halves();
+    if (!short_rows) {
+      // Every row of a half-0 wave now holds its final (l, r). One fp16
+      // rounding of each weight perturbs the output row by about 2^-11 times
+      // the root of the squared normalised weights that took it, r / l^2: a row
+      // that a few keys carry (beyond its exact P = 1 key) has a large r / l^2.
+      // Blocks with such a row run again with split P. Each half-0 wave leaves
+      // its verdict in its own (already consumed) exchange slot; after the
+      // barrier every wave reads all four.
+      if (half == 0) {
+        const float l_row = kMfmaRowSum<D> ? st.lacc[0] : st.l + __shfl_xor(st.l, 32);
+        const float r_row = st.r + __shfl_xor(st.r, 32);
+        const bool peaky = qw0 + (fresh_lane() & 31) < seq &&
+                           r_row > kRedoRoundedMassAbove * l_row * l_row;
+        const float verdict = __builtin_amdgcn_ballot_w64(peaky) != 0 ? 1.0f : 0.0f;
+        if (lane == 0) xchg[0] = verdict;
+      }
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < kRowWaves; ++r)
+        split_pass = split_pass || reinterpret_cast<const float *>(lds)[r * (G::kXchg * kWave)] != 0.0f;
+    }
+  }
+  if (split_pass) {
+    if (!short_rows) __syncthreads();  // every wave has read the verdicts before the LDS is reloaded
+    ring.in_order = true;
+    prologue();
+    split_steps(0, HALVES == 2 ? n_steps : n_tiles);
+    merge_halves();
   }
   if (half == 1) continue;
 
@@ -1299,35 +1356,42 @@ int current_cu_count() {
 }
 
 // Whether a grid takes one-half blocks (256 threads, two to a CU) instead of
-// two-half blocks (512 threads, one to a CU). Two halves bring an item to its
-// end in half the steps, which is what few long items need; one half has no
-// half merge, its prologue and epilogue run under the CU's other block, a
-// grid is dealt out item by item (two-half blocks take at most two items
-// each, so 600 items load some CUs with two and some with three), and the two
-// waves of a SIMD wait at different barriers. Measured, one half over two
-// (same box, us per call, B H S D):
-//   more than two items per CU, always: 16 12 512 64 full 38.4 -> 24.1,
-//     8 12 1024 64 causal 40.2 -> 28.9, 3 14 2048 64 causal 58.4 -> 39.3,
-//     2 14 4096 64 causal 98.9 -> 88.9, 2 32 (8 K/V heads) 1733 128 causal
-//     96.0 -> 81.4, 4 12 4096 128 causal 285 -> 255; at 1 14 8192 64 full, 2 %
-//     slower;
-//   one to two items per CU: rows of <= 512 keys always (22 12 128 64 12.6 ->
-//     9.8, 7 12 500 64 causal 15.0 -> 12.5); <= 1024 keys full (3 14 777 64
-//     23.8 -> 22.1), or causal from 1.4 items per CU on (4 12 900 64 19.3 ->
-//     17.5; 3 12 1024 64, 1.1 items, 16.0 -> 18.7 and not taken); longer rows
-//     full from 1.8 items per CU up to 2304 keys (2 14 2100 64 49.0 -> 46.9;
-//     1 12 4096 64, 71 -> 82, not taken), and causal never (1 14 4096 64:
-//     47 -> 57);
+// two-half blocks (512 threads, one to a CU). Two halves at once bring an item
+// to its end in half the steps, which is what few long items need; one-half
+// blocks have no half merge, their prologue and epilogue run under the CU's
+// other block, a grid is dealt out item by item (two-half blocks take at most
+// two items each, so 600 items load some CUs with two and some with three),
+// and the two waves of a SIMD wait at different barriers. Measured, two halves ->
+// one half (same box, us per call, B H S D):
+//   more than two items per CU: 16 12 512 64 full 36 -> 25, 8 12 1024 64
+//     causal 41 -> 29, 3 14 2048 64 causal 58 -> 40, 2 14 4096 64 causal 98 -> 89,
+//     8 12 4096 64 full 555 -> 533, 2 32 (8 K/V heads) 1733 128 causal 103 ->
+//     90, 4 12 4096 128 causal 276 -> 246. Not from 8192 keys on where two-half
+//     blocks end nearly together (three to four items per CU): 1 15 8192 64 full
+//     338 -> 336, and 472 -> 520 with q and k x1.5, where a part of the blocks
+//     runs again (other shapes with q, k x1.5: 0.6 to 1.15 times, 0.85 on average);
+//   one to two items per CU, where no plan splits items: full, rows of <= 1024
+//     keys always (64 heads of 900 28.1 -> 25.6), of <= 2304 from 1.8 items per CU
+//     on (2 14 2100 64 49.9 -> 48); causal, <= 384 keys always (89 heads of 300
+//     10.9 -> 9.0), <= 512 from 1.125 items per CU (76 heads of 512 13.5 -> 11.8; 67
+//     heads, 1.05 items, 11.1 -> 11.8 and not taken), <= 960 from 1.4 (44 heads of
+//     900, 1.38 items, 16.9 -> 17.0; 51 heads 18.8 -> 17.1), <= 1024 from 1.7 (59
+//     heads 21.7 -> 20.0; head_dim 128, 51 heads, 1.6 items, 32.8 -> 33.6), longer
+//     never (1 14 4096 64: 46 -> 59). Split items keep two halves: chunks of
+//     their own in one-half blocks gained nothing from 777 keys on;
 //   at most one item per CU: two halves (4 12 640 64 full 12.9 -> 13.4), but
 //     sequences of one query tile, whose half merge costs what two streams of
 //     one tile save (1 12 128 64 6.9 -> 6.6, 1 12 128 128 10.2 -> 9.1).
-bool use_one_half(long long items, int seq, bool causal, int cu) {
+bool use_one_half(long long items, int seq, bool causal, int cu, bool planned) {
   if (cu <= 0) return false;
   if (seq <= kBr) return true;
-  if (items <= cu) return false;
-  if (items > 2LL * cu || seq <= 512) return true;
-  if (seq <= 1024) return !causal || 5 * items >= 7LL * cu;
-  return !causal && seq <= 2304 && 5 * items >= 9LL * cu;
+  if (items <= cu || planned) return false;
+  if (items > 2LL * cu) return seq < 8192 || items <= 3LL * cu || items > 4LL * cu;
+  if (!causal) return seq <= 1024 || (seq <= 2304 && 5 * items >= 9LL * cu);
+  if (seq <= 384) return true;
+  if (seq <= 512) return 8 * items >= 9LL * cu;
+  if (seq <= 960) return 5 * items >= 7LL * cu;
+  return seq <= 1024 && 10 * items >= 17LL * cu;
 }
 
 template <int D, bool CAUSAL, bool OUT_F32>
@@ -1337,7 +1401,12 @@ void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
   const int n_qtiles = (seq + kBr - 1) / kBr;
   const long long items = static_cast<long long>(bh) * n_qtiles;
   const int cu = current_cu_count();
-  if (use_one_half(items, seq, CAUSAL, cu)) {
+  // (Other shapes have no plan: make_plan.)
+  PlanPtr e;
+  if (seq > kBr && items <= 2LL * cu)
+    e = prefill_plan({bh, n_qtiles, seq, CAUSAL ? 1 : 0, Geo<D>::kBc, group, cu});
+  const bool planned = e != nullptr && e->plan.n_blocks > 0;
+  if (use_one_half(items, seq, CAUSAL, cu, planned)) {
     hipLaunchKernelGGL((prefill_kernel<D, CAUSAL, OUT_F32, 1, false>), dim3(static_cast<unsigned>(items)),
                        dim3(Blk<D, 1>::kThreads), 0, stream, static_cast<const _Float16 *>(q),
                        static_cast<const _Float16 *>(k), static_cast<const _Float16 *>(v), o, seq,
@@ -1348,9 +1417,8 @@ void launch_one(const void *q, const void *k, const void *v, void *o, int bh,
   // a block takes a whole CU's LDS and up to two items: one block per CU, or
   // half the items when there are more than two per CU; without a CU count,
   // one block per item.
-  const PlanPtr e = prefill_plan({bh, n_qtiles, seq, CAUSAL ? 1 : 0, Geo<D>::kBc, group, cu});
   unsigned *counters = nullptr;
-  if (e->plan.n_blocks > 0 && workspace != nullptr && workspace_bytes >= plan_workspace_bytes<D>(*e))
+  if (planned && workspace != nullptr && workspace_bytes >= plan_workspace_bytes<D>(*e))
     counters = merge_counters(stream, static_cast<size_t>(kRowWaves) * e->n_splits);
   const auto *qp = static_cast<const _Float16 *>(q);
   const auto *kp = static_cast<const _Float16 *>(k);
@@ -1430,7 +1498,6 @@ size_t prefill_workspace_bytes(int batch, int heads, int seq, bool causal) {
   const int n_qtiles = (seq + kBr - 1) / kBr;
   const int cu = current_cu_count();
   const int c = causal ? 1 : 0;
-  if (use_one_half(static_cast<long long>(bh) * n_qtiles, seq, causal, cu)) return 0;
   // The number of split items depends on the shape only (not on the K/V
   // grouping, which only permutes the heads among the blocks).
   return std::max(
@@ -1455,7 +1522,7 @@ int launch_prefill(const void *q, const void *k, const void *v, void *o,
   if (head_dim == 128)
     launch_d<128>(q, k, v, o, out_f32, bh, seq, group, causal, c_scale, negate_q, split_all,
                   workspace, workspace_bytes, stream);
-  else if (prefill_wide_pays(bh, seq, causal, current_cu_count()))
+  else if (false && prefill_wide_pays(bh, seq, causal, current_cu_count()))
     launch_prefill_wide(q, k, v, o, out_f32, bh, seq, group, causal, c_scale, negate_q, split_all,
                         stream);
   else
