@@ -41,7 +41,6 @@ HIP_UNITS = [
     ("prefill_d64", "prefill.hip",
      ["-DFA_PREFILL_D=64", "-mllvm", "-amdgpu-sched-strategy=iterative-ilp"]),
     ("prefill_d128", "prefill.hip", ["-DFA_PREFILL_D=128"]),
-    ("prefill_wide", "prefill_wide.hip", []),
     ("decode", "decode.hip", []),
     ("kv_cache", "kv_cache.hip", []),
     ("legacy", "legacy.hip", []),

@@ -124,7 +124,6 @@
 // rounding: 3.8e-7 to 2.8e-5 at 512 keys with q and k x1.5.)
 
 #include <algorithm>
-#include <climits>
 #include <map>
 #include <memory>
 #include <mutex>
@@ -134,7 +133,6 @@
 
 #include "fa_internal.h"
 #include "mfma_tile.h"
-#include "prefill_common.h"
 
 // This file is compiled once per head size: FA_PREFILL_D = 64 gives the
 // head_dim 64 kernels and the shared host entry points, FA_PREFILL_D = 128
@@ -155,6 +153,24 @@ constexpr int kVStages = 5;
 constexpr int kAhead = 4;                     // tiles in flight ahead of use
 constexpr float kCarryMax = 64.0f;            // log2 units (one-half blocks, see main_steps)
 constexpr int kLoadsPerTile = 4;              // global_load_lds per thread per tile
+constexpr int kSplitPRowsBelow = 256;  // rows with fewer keys than this: split P
+// A block is recomputed with split P when, for one of its rows, the squared
+// normalised weights that took a single fp16 rounding sum to more than this
+// (see the precision note at the top of the file).
+constexpr float kRedoRoundedMassAbove = 0.03f;
+// |scale| * sqrt(D) above this (1 is the standard 1/sqrt(D)): rows are peaky
+// from the scale alone, so the first (single-rounding) pass is skipped.
+[[maybe_unused]] constexpr float kSplitAllWidth = 1.5f;  // used by the head_dim 64 build
+constexpr float kNegHuge = -3.0e38f;
+// The max that P is taken against moves only when a row's tile max exceeds it
+// by more than this (log2 units), so P <= 2^8 and O is rescaled on few steps...
+constexpr float kLazyMaxSlack = 8.0f;
+// ...or when the tile max's weight exceeds this fraction of the row sum so
+// far: a key that carries a large share of its row is then taken at the exact
+// max, where its P = 1 is exact and leaves the rounded mass.
+constexpr float kLazyMaxDominant = 1.0f / 16;
+constexpr int kLazyMaxRowsFrom = 1024;  // keys a row sees (at least) to take the lazy max
+
 // Tile geometry for head_dim D (64 or 128). A K or V tile is always 8 KiB:
 // 64 keys of 128 B rows for D = 64, 32 keys of 256 B rows for D = 128, so a
 // step is 16 MFMAs either way (D = 64: QK 2 key blocks x 4 d-steps, PV 4
@@ -203,6 +219,20 @@ struct Blk : Geo<D> {
 
 [[maybe_unused]] __device__ __forceinline__ half8 lds_b128(const _Float16 *p) {
   return *reinterpret_cast<const half8 *>(p);
+}
+
+// The lane index read afresh from the hardware (v_mbcnt, in volatile asm so
+// that the compiler cannot merge it with the kernel's first lane index). The
+// code after the main loop (masked tail, verdict, epilogue) derives its
+// per-lane values from this instead of from values computed before the loop,
+// which the compiler otherwise keeps live across it: at 256 VGPRs they went
+// to scratch (5 per lane at head_dim 64, 11-15 at 128), each item stored and
+// reloaded them, and their write-backs were 2.5-3.4 MB of a C3 launch's HBM
+// writes (C3 46.2 -> 45.8 us, C2 full 27.1 -> 26.4 us without them).
+__device__ __forceinline__ int fresh_lane() {
+  int l;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(l));
+  return l;
 }
 
 // head_dim 64 sums P rows on the matrix cores (rowsum_mfma); head_dim 128,
@@ -580,6 +610,50 @@ struct HalfRing {
     issue(k + kAhead);
   }
 };
+
+// Block -> (b, h) with XCD affinity. The grid stays in level-major order
+// (every head's heaviest query tile first), and blocks go to the 8 XCDs
+// round-robin (block i on XCD i % 8). Head h is "at home" on XCD h % 8:
+// within a level each XCD fills its positions with its home heads first and
+// the leftover heads take the spare positions in a fixed order, so most of a
+// head's blocks share one XCD's L2 (for 14 heads, 89 % of the blocks).
+__host__ __device__ __forceinline__ int home_head(int i, int n_bh) {
+  const int level = i / n_bh;
+  const int k = i - level * n_bh;
+  const int base = (level * n_bh) & 7;
+  const int x = (base + k) & 7;     // XCD of this block
+  const int d_x = (x - base) & 7;   // first position of XCD x in this level
+  const int r = (k - d_x) >> 3;     // rank of position k among XCD x's
+  const int nhome_x = (n_bh - x + 7) >> 3;
+  if (r < nhome_x) return x + 8 * r;
+  // A spare position: its index among all spares (XCDs in order, then rank)
+  // selects the matching overflow head (XCDs in order, then head rank).
+  int s = r - nhome_x;
+  for (int y = 0; y < x; ++y) {
+    const int npos = (n_bh - ((y - base) & 7) + 7) >> 3;
+    const int nhome = (n_bh - y + 7) >> 3;
+    s += npos > nhome ? npos - nhome : 0;
+  }
+  for (int y = 0; y < 8; ++y) {
+    const int npos = (n_bh - ((y - base) & 7) + 7) >> 3;
+    const int nhome = (n_bh - y + 7) >> 3;
+    const int over = nhome > npos ? nhome - npos : 0;
+    if (s < over) return y + 8 * (npos + s);
+    s -= over;
+  }
+  return 0;  // unreachable: spare positions and overflow heads are equal in number
+}
+
+// Grouped queries: the placement heads of XCD x (x, x + 8, x + 16, ...) are
+// given a contiguous run of query heads, in XCD order, so the query heads
+// that read one K/V head (consecutive indices) mostly share an XCD and its
+// L2 holds one copy of that K/V head.
+__host__ __device__ __forceinline__ int grouped_head(int h, int n_bh) {
+  const int x = h & 7;
+  int start = 0;
+  for (int y = 0; y < x; ++y) start += (n_bh - y + 7) >> 3;
+  return start + (h >> 3);
+}
 
 // Work units and their blocks, planned on the host when the items do not
 // fill the chip evenly (at most two per CU): the heaviest items are split
@@ -1522,9 +1596,6 @@ int launch_prefill(const void *q, const void *k, const void *v, void *o,
   if (head_dim == 128)
     launch_d<128>(q, k, v, o, out_f32, bh, seq, group, causal, c_scale, negate_q, split_all,
                   workspace, workspace_bytes, stream);
-  else if (false && prefill_wide_pays(bh, seq, causal, current_cu_count()))
-    launch_prefill_wide(q, k, v, o, out_f32, bh, seq, group, causal, c_scale, negate_q, split_all,
-                        stream);
   else
     launch_d<64>(q, k, v, o, out_f32, bh, seq, group, causal, c_scale, negate_q, split_all,
                  workspace, workspace_bytes, stream);

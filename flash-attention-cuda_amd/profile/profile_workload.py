@@ -40,7 +40,7 @@ WORKLOADS = {
                           "flop", 4.0 * 4 * 12 * 1024 * 1024 * 64 / 2),
     "prefill_c2_full": ("config 2: full prefill B=4 H=12 S=1024", "prefill_kernel<64, false",
                         "flop", 4.0 * 4 * 12 * 1024 * 1024 * 64),
-    "prefill_large": ("full prefill B=8 H=12 S=4096 (64-row waves)", "prefill_wide_kernel<false",
+    "prefill_large": ("full prefill B=8 H=12 S=4096 (one-half blocks)", "prefill_kernel<64, false",
                       "flop", 4.0 * 8 * 12 * 4096 * 4096 * 64),
     "prefill_c3_d128": ("config 3 shape at head_dim 128: causal prefill B=1 H=14 S=4096 D=128, scale 1/sqrt(128)",
                         "prefill_kernel<128, true", "flop", 4.0 * 14 * 4096 * 4096 * 128 / 2),

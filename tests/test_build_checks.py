@@ -60,10 +60,3 @@ def test_kernels_touch_m0_only_in_their_global_load_lds_sequences():
         assert "global_load_lds_dwordx4" in text, src
         problems = fa_build.m0_problems(text)
         assert not problems, f"{src}: " + "; ".join(problems[:5])
-
-
-def test_wide_prefill_touches_m0_only_in_its_global_load_lds_sequences():
-    with tempfile.TemporaryDirectory() as tmp:
-        text = fa_build.device_assembly("prefill_wide", tmp)
-    assert "global_load_lds_dwordx4" in text
-    assert not fa_build.m0_problems(text)

@@ -1,7 +1,7 @@
 """Prefill grids of more than one 128-row item per CU: one-half blocks
-(csrc/prefill.hip, use_one_half) and, at head_dim 64, 256-row blocks
-(csrc/prefill_wide.hip, prefill_wide_pays): every place a ragged end or the
-causal diagonal can fall in a block's tiles, against the oracle."""
+(csrc/prefill.hip, use_one_half): every place a ragged end or the causal
+diagonal can fall in a block's tiles, against the oracle, and their rounding
+against that of two-half blocks."""
 
 import ctypes
 import math
@@ -141,28 +141,22 @@ def test_one_half_blocks_moving_max(kind, causal, d):
     assert err <= BOUND, err
 
 
-def _wide_case(seq, causal):
-    """Heads that give a grid the 256-row blocks take, and heads to check."""
-    cu = torch.cuda.get_device_properties(0).multi_processor_count
-    tiles = -(-seq // 256)
-    heads = 5 * cu // tiles + 1 if causal else 2 * cu // tiles
-    return heads - heads % 2, [0, 1, heads // 3, heads // 2, heads - 3]
-
-
+@pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("causal,seq", [
-    *[(False, s) for s in (512, 513, 544, 575, 577, 608, 639, 700, 768)],
-    *[(True, s) for s in (2048, 2049, 2079, 2111, 2145, 2240)],
+    *[(False, s) for s in (512, 513, 544, 575, 577, 608, 639, 700, 768, 1024, 1100, 2090)],
+    *[(True, s) for s in (1024, 1100, 2048, 2049, 2079, 2111, 2145, 2240)],
 ])
-def test_wide_blocks_at_every_tail(seq, causal):
-    heads, check = _wide_case(seq, causal)
-    _check_prefill(1, heads, heads, seq, 64, causal, 0.125, check=check)
+def test_one_half_blocks_at_every_tail_of_long_rows(seq, causal, d):
+    heads = _heads_for(seq, 2)
+    _check_prefill(1, heads, heads, seq, d, causal, d ** -0.5, check=[0, heads // 2, heads - 1])
 
 
+@pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("kind", ["grouped", "negative scale", "wide scale", "wide inputs"])
-def test_wide_blocks_options(kind, causal):
-    seq = 2090 if causal else 720
-    heads, check = _wide_case(seq, causal)
-    scale = {"negative scale": -0.125, "wide scale": 0.3}.get(kind, 0.125)
-    _check_prefill(1, heads, heads // 2 if kind == "grouped" else heads, seq, 64, causal, scale,
-                   1.5 if kind == "wide inputs" else 1.0, check)
+def test_one_half_blocks_options_on_long_rows(kind, causal, d):
+    seq = 2090 if causal else 1100
+    heads = 2 * (_heads_for(seq, 2) // 2 + 1)
+    scale = {"negative scale": -1.0, "wide scale": 2.4}.get(kind, 1.0) * d ** -0.5
+    _check_prefill(1, heads, heads // 2 if kind == "grouped" else heads, seq, d, causal, scale,
+                   1.5 if kind == "wide inputs" else 1.0, [0, 1, heads // 2, heads - 1])
