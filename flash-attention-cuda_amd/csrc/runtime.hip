@@ -277,7 +277,8 @@ size_t decode_workspace_impl(int batch, int heads, int kv_heads, int max_seq, in
 }
 
 // scratch_ws: the workspace is the library's own per-device scratch
-// (fa_decode_hd_noalloc), which only changes the message of a size failure.
+// (fa_decode_hd_noalloc), which changes the message of a size failure and, for
+// grouped calls, the automatic chunk where its partials would not fit.
 int decode_impl(const void *q, const void *k_cache, const void *v_cache,
                 const int32_t *seq_lens, void *o, int out_dtype, int batch, int heads,
                 int kv_heads, int max_seq, int head_dim, float scale, int split_size,
@@ -311,8 +312,9 @@ int decode_impl(const void *q, const void *k_cache, const void *v_cache,
   rc = resolve_split(batch, heads, kv_heads, max_seq, head_dim, &split_size);
   if (rc != FA_OK) return rc;
   // The fixed scratch takes every grouped shape that fits it at chunks of 160
-  // rows, also where the automatic choice is 128.
-  if (scratch_ws && auto_split && kv_heads != heads && split_size < 160 && max_seq > 160 &&
+  // rows, also where the automatic choice is 128 (caches of 129 to 160 rows
+  // among them: one chunk instead of two).
+  if (scratch_ws && auto_split && kv_heads != heads && split_size < 160 && max_seq > split_size &&
       decode_ws_bytes(batch, heads, max_seq, head_dim, split_size) > workspace_bytes)
     split_size = 160;
   const size_t n_splits = (static_cast<size_t>(max_seq) + split_size - 1) / split_size;

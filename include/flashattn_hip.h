@@ -222,7 +222,8 @@ int fa_kv_append_hd(void *k_cache, void *v_cache, const void *k_new,
  * FA_NOALLOC_SCRATCH_BYTES that the library holds on every device it runs on
  * until the process ends. A shape whose partials need more fails with
  * FA_ERR_WORKSPACE before anything is launched (fa_decode_hd_workspace_bytes
- * gives the need). Every call on one device shares that device's array and
+ * gives the need; a grouped call with split_size 0 whose automatic chunk does
+ * not fit runs with chunks of 160 rows if those do). Every call on one device shares that device's array and
  * leaves its contents behind: calls that overlap in time on one device
  * (several streams or threads) race, so the caller must serialise them.
  * Same arguments, rules and results as fa_decode_hd otherwise. */

@@ -164,3 +164,14 @@ def test_noalloc_grouped_takes_longer_chunks_where_the_automatic_ones_do_not_fit
     got = _run(lib, True, q, k, v, lens, FA_OUT_F32, 1, 0.125, 0)
     want = _run(lib, False, q, k, v, lens, FA_OUT_F32, 1, 0.125, 160)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("max_seq", [129, 140, 150])
+def test_noalloc_grouped_takes_short_caches_as_one_chunk(lib, max_seq):
+    """Caches of a little over 128 rows: two automatic 128-row chunks need 14.7 MB of
+    partials, one 160-row chunk 7.4 MB: the call runs with that."""
+    q, k, v, lens = _inputs(218, 128, 4, max_seq, 64, seed=max_seq)
+    assert lib.fa_decode_hd_workspace_bytes(218, 128, 4, max_seq, 64, 0) > SCRATCH_BYTES
+    got = _run(lib, True, q, k, v, lens, FA_OUT_F32, 4, 0.125, 0)
+    want = _run(lib, False, q, k, v, lens, FA_OUT_F32, 4, 0.125, 160)
+    assert torch.equal(got, want)
