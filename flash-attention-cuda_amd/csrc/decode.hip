@@ -1300,14 +1300,16 @@ int decode_group_chunk(int batch, int units_per_row, int max_seq, int head_dim) 
   // chunk adds a partial to merge. head_dim 64: 1.25x the share (us per call,
   // chunk: B32 H14/2 L4096 ragged 160 rows 14.2, 256 12.7, 512 14.7; B1 H14/2
   // L4096 96 rows 7.0, 128 7.0, 160 7.5, 256 9.1; B32 H32/8 L4096 640 31.5, 1024
-  // 30.8). head_dim 128: 1.5x a share of up to 384 rows (B1 H32/8 L16384 192
-  // rows 17.9, 256 16.2, 384 17.8; B2 H32/8 L16384 all full 352 26.4, 512
-  // 25.4; B1 H28/4 L16384 96 14.9, 128 12.9), else the share (B8 H32/8 L8191
-  // ragged 704 32.1, 1024 32.3, all full 45.9, 44.1).
+  // 30.8). head_dim 128: the share, or 1.5x of one of up to 320 rows for one or
+  // two sequences, whose waves leave the chip together (B1 H32/8 L16384 192 rows
+  // 15.9, 224 16.7, 256 15.1; L30000 320 rows 23.8, 416 26.1, 480 23.6; B2 H32/8
+  // L18432 384 rows 27.2, 480 29.1, 576 28.4; ragged batches wait for their longest
+  // chunk: B8 H32/8 L3600 320 rows 16.8, 384 18.5, 480 18.3, L4096 352 18.6, 544
+  // 20.0). Nothing between the share and 1.5x of it pays, so the rule has a step.
   long long rows = (work + waves - 1) / waves;
   if (head_dim != 128)
     rows = (5 * work + 4 * waves - 1) / (4 * waves);
-  else if (rows <= 384)
+  else if (batch <= 2 && rows <= 320)
     rows += rows / 2;
   rows = ((rows + kGroupTile - 1) / kGroupTile) * kGroupTile;
   const long long cap = ((static_cast<long long>(max_seq) + kGroupTile - 1) / kGroupTile) * kGroupTile;
