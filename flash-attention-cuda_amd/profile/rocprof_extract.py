@@ -365,8 +365,12 @@ def render_bench(report: dict, command: str = "") -> str:
 
 
 def render_occupancy(report: dict, command: str = "") -> str:
-    lines = ["# Theoretical occupancy of every kernel (occupancy_report())", ""]
+    lines = ["# Theoretical occupancy of the kernels (occupancy_report())", ""]
     lines += _header(command)
+    lines += ["One launch shape of each kernel: `prefill_kernel` in two-half blocks without a plan "
+              "(large grids run 256-thread blocks, two to a CU), `decode_merge_kernel` with 4 waves "
+              "(1 to 16 by the number of chunks), `decode_group_kernel` for up to 16 query heads per "
+              "K/V head.", ""]
     lines += ["| kernel | threads/block | VGPRs/thread | LDS/block | blocks/CU | occupancy |",
               "| :-- | ---: | ---: | ---: | ---: | ---: |"]
     for row in report.get("occupancy", []):

@@ -116,7 +116,9 @@ def render(device, occupancy, prefill, before, after, adaptive, command):
 
     w("## Kernel resources and theoretical occupancy")
     w("")
-    w("From `flashattn_cuda.occupancy_report()` at each kernel's launch configuration.")
+    w("From `flashattn_cuda.occupancy_report()`, one launch shape of each kernel: `prefill_kernel`")
+    w("in two-half blocks without a plan, `decode_merge_kernel` with 4 waves, `decode_group_kernel`")
+    w("for up to 16 query heads per K/V head.")
     w("")
     w("| kernel | threads/block | registers/thread | LDS/block | max blocks/CU | theoretical occupancy |")
     w("| :-- | ---: | ---: | ---: | ---: | ---: |")
@@ -125,8 +127,9 @@ def render(device, occupancy, prefill, before, after, adaptive, command):
           f"{row['shared_bytes_per_block']:,} B | {row['max_active_blocks_per_sm']} | "
           f"{row['theoretical_occupancy'] * 100:.1f}% |")
     w("")
-    w("The prefill block is one per CU by design (8 waves, 160 KiB of LDS rings): two waves")
-    w("per SIMD, the pairing that lets one wave's MFMAs run under the other's softmax.")
+    w("The two-half prefill block is one per CU by design (8 waves, 160 KiB of LDS rings): two")
+    w("waves per SIMD, the pairing that lets one wave's MFMAs run under the other's softmax. Large")
+    w("grids run blocks of 4 waves and 72 KiB, two per CU, for the same two waves per SIMD.")
     w("")
 
     w("## Prefill roofline")

@@ -252,7 +252,11 @@ int fa_legacy_attention(const float *q, const float *k, const float *v,
                         float *o, int n, int variant, void *stream);
 
 /* Fill up to `capacity` entries (one per kernel) for the current device;
- * *count receives the number of kernels. Returns an fa_status. */
+ * *count receives the number of kernels. Each entry is one launch shape of its
+ * kernel: prefill_kernel in two-half blocks of 512 threads without a plan (large
+ * grids run blocks of 256 threads, two to a compute unit), decode_merge_kernel
+ * with 4 waves (1 to 16 by the number of chunks), decode_group_kernel for up to
+ * 16 query heads per K/V head. Returns an fa_status. */
 int fa_occupancy_report(fa_occupancy_entry *out, int capacity, int *count);
 
 #ifdef __cplusplus
