@@ -1295,9 +1295,13 @@ int decode_group_chunk(int batch, int units_per_row, int max_seq, int head_dim) 
       head_dim == 128 ? GroupGeo<128>::kWavesPerCu : GroupGeo<64>::kWavesPerCu;
   const long long waves = static_cast<long long>(per_cu) * (cu > 0 ? cu : 256);
   const long long work = static_cast<long long>(max_seq) * batch * units_per_row;
-  // Chunks of at least 128 rows, and longer than the one-round share where
-  // that is short: a wave's first tile arrives ~2 us after it starts and every
-  // chunk adds a partial to merge. head_dim 64: 1.25x the share (us per call,
+  // Chunks of at least 128 rows (head_dim 128, caches of up to 4096 rows, 64
+  // chunks and half a round of the merge: 64), and longer than the one-round share
+  // where that is short: a wave's first tile arrives ~2 us after it starts and
+  // every chunk adds a partial to merge. Minimum, head_dim 128, us of the two
+  // kernels with chunks of 64 / 128 rows: B1 H8/4 L300 6.5 / 8.0, B1 H14/2 L4096
+  // 7.1 / 8.3, B1 H28/4 L8000 9.0 / 8.9, B1 H2/1 L30000 12.8 / 11.0; per call 96
+  // / 128, B4 H64/2 L8192 15.6 / 14.7. head_dim 64: 1.25x the share (us per call,
   // chunk: B32 H14/2 L4096 ragged 160 rows 14.2, 256 12.7, 512 14.7; B1 H14/2
   // L4096 96 rows 7.0, 128 7.0, 160 7.5, 256 9.1; B32 H32/8 L4096 640 31.5, 1024
   // 30.8). head_dim 128: the share, or 1.5x of one of up to 320 rows for one or
@@ -1313,7 +1317,8 @@ int decode_group_chunk(int batch, int units_per_row, int max_seq, int head_dim) 
     rows += rows / 2;
   rows = ((rows + kGroupTile - 1) / kGroupTile) * kGroupTile;
   const long long cap = ((static_cast<long long>(max_seq) + kGroupTile - 1) / kGroupTile) * kGroupTile;
-  rows = std::max<long long>(rows, 4 * kGroupTile);
+  const int min_tiles = head_dim == 128 && max_seq <= 4096 ? 2 : 4;
+  rows = std::max<long long>(rows, min_tiles * kGroupTile);
   return static_cast<int>(std::min(rows, std::max<long long>(cap, 2 * kGroupTile)));
 }
 

@@ -75,7 +75,7 @@ unsigned *merge_counters(hipStream_t stream, size_t n);
 int decode_units_per_row(int heads, int kv_heads);
 // Automatic chunk (cache rows per split) of the grouped-query decode pass:
 // the batch's max_seq-row work over the waves the GPU runs at once, in
-// multiples of 32 rows, at least 128 (as many as the cache has).
+// multiples of 32 rows, at least 64 or 128 (as many as the cache has).
 int decode_group_chunk(int batch, int units_per_row, int max_seq, int head_dim);
 
 // Writes k_new / v_new ([B, H_kv, 1, 64]) at row seq_lens[b] of the caches
