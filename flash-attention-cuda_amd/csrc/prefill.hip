@@ -387,7 +387,8 @@ __device__ __forceinline__ bool tile_max(floatx16 (&s)[Geo<D>::kKB], int lim, fl
   float mx_c;
   {
     // No contraction: with mx_c rounded once, a tile that sets m gets
-    // largest weight exp2(0) = 1 exactly.
+    // pm = exp2(0) = 1 exactly (the weight itself, from the unrounded
+    // product, rounds to 1 in fp16).
 #pragma clang fp contract(off)
     mx_c = mx * c_scale;
   }
