@@ -39,9 +39,13 @@ def _check_prefill(batch, heads, kv_heads, seq, d, causal, scale, spread=1.0, ch
 
 
 def _heads_for(seq, per_cu):
-    """Query heads of one sequence that give more than per_cu items per CU."""
+    """Query heads of one sequence that give more than per_cu items per CU
+    (above two, and below 8192 keys, use_one_half takes every grid)."""
     cu = torch.cuda.get_device_properties(0).multi_processor_count
-    return int(per_cu * cu) // -(-seq // 128) + 1
+    tiles = -(-seq // 128)
+    heads = int(per_cu * cu) // tiles + 1
+    assert heads * tiles > per_cu * cu and seq < 8192
+    return heads
 
 
 @pytest.mark.parametrize("d", [64, 128])
